@@ -402,6 +402,7 @@ def run(st):
     if st.kind == "chains":
         for t in st.trees:
             pf.p4_setPrams(t.cTree, -1)
+            pf.markAll(t.cTree, -1)
         lnLs = st.batch.logLikes()
         return lnLs, numpy.stack([t.partLikes for t in st.trees])
     if st.kind == "moves":
