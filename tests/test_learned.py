@@ -133,6 +133,34 @@ def test_gradients_match_oracle():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("f,h,o,n", [(1, 16, 2, 1), (31, 64, 6, 15), (33, 65, 8, 16), (64, 80, 34, 17), (24, 256, 6, 1025),
+                                     (512, 512, 64, 33), (24, 513, 6, 40), (513, 32, 6, 40)])
+def test_every_width_matches_oracle(f, h, o, n):
+    """Widths at and around the padding steps and limits of the fused
+    kernels, and beyond them (one kernel per product); the tolerances of
+    test_forward_matches_oracle and test_gradients_match_oracle."""
+    rng = numpy.random.default_rng(f + h + o + n)
+    net = pf.Mlp(f, h, o, seed=8)
+    th = (net.getParams() + 0.05 * rng.normal(size=net.nParams)).astype(numpy.float32)
+    net.setParams(th)
+    X, Y, M = _batch(rng, n, f, o // 2)
+    X *= 1.0 / math.sqrt(f)
+    ref, _ = mo.forward(th, X, f, h, o, bf16=True)
+    assert numpy.abs(net.forward(X) - ref).max() < 3e-4 * max(1.0, numpy.abs(ref).max())
+    L, g = net.gradients(X, Y, M)
+    Lo, go = mo.loss_and_grad(th, X, Y, M, f, h, o, bf16=True)
+    assert abs(L - Lo) < 1e-4 * abs(Lo)
+    assert numpy.linalg.norm(g - go) < 2e-3 * numpy.linalg.norm(go)
+    # a step after a change of batch size, on the same handle
+    assert net.trainStep(X, Y, M, 1e-3) == L
+    want, _, _ = mo.adam_step(th.astype(float), g.astype(float), numpy.zeros(net.nParams), numpy.zeros(net.nParams), 1, 1e-3)
+    new = net.getParams()
+    assert numpy.abs(new - want).max() < 2e-6
+    ref, _ = mo.forward(new.astype(float), X, f, h, o, bf16=True)
+    assert numpy.abs(net.forward(X) - ref).max() < 3e-4 * max(1.0, numpy.abs(ref).max())
+
+
+@pytest.mark.gpu
 def test_train_step_is_adam_on_the_gradients():
     rng = numpy.random.default_rng(5)
     net = pf.Mlp(F, H, O, seed=5)
