@@ -179,7 +179,7 @@ int p4g_treeLogLike(p4g_tree *t, int getSiteLikes, double *lnL);
  * harnesses that forbid hipMalloc): p4g_treeLogLike(t, 0, lnL) computed with
  * no allocation.  The pruning kernels' reduction scratch (per-workgroup sums,
  * bad-site flags, the ticket counter) comes from one library-wide device
- * array of 512 KiB per GPU instead of the tree's own buffers; a part needing
+ * array per GPU instead of the tree's own buffers; a part needing
  * more (more than about 43,000 pattern tiles, some 700,000 patterns) is
  * rejected with an error.  The tree must already hold device state for its
  * current precision (one earlier p4g_treeLogLike, which allocates);
@@ -369,12 +369,12 @@ void p4g_setPruneTuning(int fp32, int opsPerGroup, int stagePInLds);
  * eigensystem.  Takes effect at the next flush of pending P matrices;
  * eigensystems skipped meanwhile are recomputed when needed. */
 void p4g_setPmatRoute(int direct);
-/* Layout of the 20-state FP32 (MFMA) pruning launch (no counterpart in the
- * reference): with categoryWaves = 1 (the default) a program of at least
- * minOps node ops (default 32: full evaluations, not short dirty paths)
- * runs one wavefront per (16-pattern tile, gamma category), with one
- * barrier per op; otherwise one wavefront per tile holds every category.
- * Partials are the same either way. */
+/* Kept from the time when 20-state FP32 programs of at least minOps node ops
+ * ran on a kernel of their own: one kernel now serves every 20-state program
+ * of either precision, with one wavefront per (16-pattern tile, gamma
+ * category), and the results do not depend on these.  They still decide from
+ * which size on p4g_treeLogLikeNoAlloc refuses a 20-state FP32 part (one
+ * workgroup per 16 patterns counted for such programs, per 64 otherwise). */
 void p4g_setAaTuning(int categoryWaves, int minOps);
 /* LDS cap for the 4-state program's preloaded clean children (no
  * counterpart in the reference): a dirty-path program preloads the clean
@@ -383,10 +383,10 @@ void p4g_setAaTuning(int categoryWaves, int minOps);
  * from HBM when used), keeping the occupancy of full programs; 0 (the
  * default) lets preloads fill the LDS budget. */
 void p4g_setWavePreloadLds(int bytes);
-/* LDS slot file of the 20-state category-wave kernel (no counterpart in the
- * reference): its programs run in Sethi-Ullman order and forward up to
- * maxSlots children per workgroup through LDS instead of re-reading them
- * from HBM (default 5; 0 turns forwarding off).  Same partials either way. */
+/* LDS slot file of the 20-state kernel (no counterpart in the reference):
+ * its programs run in Sethi-Ullman order and forward up to maxSlots children
+ * per workgroup through LDS instead of re-reading them from HBM (default 5; 0
+ * turns forwarding off).  Same partials either way. */
 void p4g_setAaLdsSlots(int maxSlots);
 double p4g_lastKernelMicroseconds(const p4g_tree *t);
 

@@ -39,7 +39,8 @@ __device__ __forceinline__ double ancClAt(const AncArgs &a, int slot, int k, int
     if (a.layout == CL_WAVE)
         o = (((size_t)k * nPP) + p) * 4 + j;
     else if (a.layout == CL_TILED)
-        o = (size_t)(p / 16) * a.K * 320 + (((size_t)k * 5 + j / 4) * 4 + j % 4) * 16 + p % 16;
+        o = (size_t)(p / AA_TILE) * (a.K * aaPartBytes(a.fp32) / (a.fp32 ? 4 : 8)) + (size_t)k * AA_PART +
+            aaIndex(j, p % AA_TILE, a.fp32 != 0);
     else
         o = ((size_t)p * a.K + k) * a.dim + j;
     const char *base = (const char *)a.cl + a.slotBytes * slot;
@@ -48,6 +49,10 @@ __device__ __forceinline__ double ancClAt(const AncArgs &a, int slot, int k, int
 __device__ __forceinline__ int ancExpAt(const AncArgs &a, int slot, int k, int p)
 {
     if (!a.fp32) return 0;
+    if (a.layout == CL_TILED) {
+        const char *tile = (const char *)a.cl + a.slotBytes * slot + (size_t)(p / AA_TILE) * a.K * aaPartBytes(true);
+        return ((const int *)(tile + (size_t)a.K * AA_PART * 4))[k * AA_TILE + p % AA_TILE];
+    }
     const size_t o = a.layout == CL_WAVE ? (size_t)k * a.nPatPad + p : (size_t)p;
     return a.scl[(size_t)slot * a.sclPerSlot + o];
 }

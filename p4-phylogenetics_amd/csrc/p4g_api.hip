@@ -47,8 +47,10 @@ static int g_devState = 0;  // 0 unknown, 1 ready, -1 unavailable
 // buffers.  Every GPU holds its own copy of the array until the process
 // ends; host code uses the device address that hipGetSymbolAddress returns
 // for the current device (g_scratch), never the array's name.
-constexpr size_t NOALLOC_SCRATCH_BYTES = 512 * 1024;
-static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
+constexpr size_t NOALLOC_SCRATCH_BYTES = 512 * 1024;   // the limit of one part
+// (20-state parts count fewer, larger workgroups against the limit than
+// their kernel has: at most one per 256 patterns where it has one per 16)
+static __device__ __align__(256) unsigned char scratch[16 * NOALLOC_SCRATCH_BYTES];
 constexpr int MAX_DEVICES = 64;
 static unsigned char *g_scratch[MAX_DEVICES] = {};
 
@@ -162,6 +164,8 @@ static void freeTreePart(TreePart &t)
     devFree(t.eigLam);
     devFree(t.PT64);
     devFree(t.PT32);
+    if (t.PA) (void)hipFree(t.PA);
+    t.PA = nullptr;
     if (t.cl) (void)hipFree(t.cl);
     t.cl = nullptr;
     if (t.PP) (void)hipFree(t.PP);
@@ -396,6 +400,8 @@ static bool allocTreePart(Tree *t, int pNum)
         if (tp.cl) (void)hipFree(tp.cl);
         tp.cl = nullptr;
         devFree(tp.scl);
+        if (tp.PA) (void)hipFree(tp.PA);
+        tp.PA = nullptr;
         // the block count depends on the kernel
         devFree(tp.blockSums);
         devFree(tp.blockBad);
@@ -416,6 +422,7 @@ static bool allocTreePart(Tree *t, int pNum)
     tp.nPatPad = dp->dev.nPatPad;
     tp.precision = t->precision;
     tp.wave = wave;
+    tp.mfma = pruneUsesMfma(S, K, t->precision);
     tp.sclPerSlot = (size_t)(wave ? K : 1) * tp.nPatPad;
     // slots: every non-leaf node, plus one for a leaf root
     t->slotOf.assign(t->nNodes, -1);
@@ -430,22 +437,27 @@ static bool allocTreePart(Tree *t, int pNum)
     const size_t nPS = (size_t)t->nNodes * K * S * S;
     // blocks of the launch: the largest count any pruning kernel may use
     // enough block sums for any kernel choice (the smallest tile: 16 patterns)
-    tp.maxBlocks = tp.nPatPad / std::min({pruneBlockPatternsFor(S, K, t->precision, 0), pruneBlockPatterns(K), 16});
+    tp.maxBlocks = tp.nPatPad / std::min(pruneBlockPatterns(K), AA_TILE);
     const size_t elt = t->precision == FP32 ? sizeof(float) : sizeof(double);
-    tp.clBytes = (size_t)tp.nPatPad * K * S * elt;
+    tp.clBytes = tp.mfma ? (size_t)(tp.nPatPad / AA_TILE) * K * aaPartBytes(t->precision == FP32)
+                         : (size_t)tp.nPatPad * K * S * elt;
     if (!devAlloc(&tp.eigV, (size_t)tp.nEig * S * S, "hipMalloc eigV") ||
         !devAlloc(&tp.eigVi, (size_t)tp.nEig * S * S, "hipMalloc eigVi") ||
         !devAlloc(&tp.eigLam, (size_t)tp.nEig * S, "hipMalloc eigLam") ||
-        !devAlloc(&tp.PT64, nPS, "hipMalloc P64") || !devAlloc(&tp.PT32, nPS, "hipMalloc P32") ||
+        !devAlloc(&tp.PT64, nPS, "hipMalloc P64") ||
+        (!tp.mfma && !devAlloc(&tp.PT32, nPS, "hipMalloc P32")) ||
         !devAlloc(&tp.blockSums, tp.maxBlocks, "hipMalloc blockSums") ||
         !devAlloc(&tp.blockBad, tp.maxBlocks, "hipMalloc blockBad") ||
         !devAlloc(&tp.counter, 1, "hipMalloc counter") ||
         !devAlloc(&tp.patLikes, tp.nPatPad, "hipMalloc patLikes"))
         return false;
+    if (tp.mfma && !tp.PA &&
+        !hipOk(hipMalloc(&tp.PA, elt * aaMatStride(t->precision == FP32) * (size_t)t->nNodes * K), "hipMalloc P operands"))
+        return false;
     if (!tp.cl && !hipOk(hipMalloc(&tp.cl, tp.clBytes * tp.nSlots), "hipMalloc partials")) return false;
     if (!tp.PP && !hipOk(hipMalloc(&tp.PP, (size_t)K * t->nNodes * 16 * sizeof(double)), "hipMalloc staged P"))
         return false;
-    if (t->precision == FP32 && !devAlloc(&tp.scl, (size_t)tp.nSlots * tp.sclPerSlot, "hipMalloc scale"))
+    if (t->precision == FP32 && !tp.mfma && !devAlloc(&tp.scl, (size_t)tp.nSlots * tp.sclPerSlot, "hipMalloc scale"))
         return false;
     if (!tp.hArena) {
         auto up16 = [](size_t b) { return (b + 15) & ~(size_t)15; };
@@ -673,7 +685,8 @@ static bool launchParams(Tree *t, int pNum, std::vector<DeferredP> *defer = null
         const char *d = (devEig ? (const char *)tp.dArena : base) + tp.offPack;
         PmatArgs a{S, K, nI, reinterpret_cast<const int *>(d + sizeof(double) * nI * K),
                    reinterpret_cast<const int *>(d + sizeof(double) * nI * K + sizeof(int) * nI),
-                   reinterpret_cast<const double *>(d), tp.eigV, tp.eigVi, tp.eigLam, tp.PT64, tp.PT32};
+                   reinterpret_cast<const double *>(d), tp.eigV, tp.eigVi, tp.eigLam, tp.PT64, tp.PT32,
+                   tp.PA, t->precision == FP32 ? 1 : 0};
         const double *inDev = devEig ? reinterpret_cast<const double *>(tp.dArena) : nullptr;
         if (direct && defer) {
             defer->push_back({a, reinterpret_cast<const double *>(base), inDev});
@@ -882,7 +895,8 @@ static uint64_t programKey(const Tree *t, int pNum, bool full)
     mix(pruneWaveVectorP(t->precision));
     mix(pruneWaveLean(t->precision));
     mix(pruneGroupWidthFor(tp.dim, t->precision));
-    mix(pruneAaLdsSlots(tp.K));
+    mix(tp.mfma);
+    mix(pruneAaLdsSlots(tp.K, t->precision));
     mix(pruneWavePreloadSlots(tp.K, 1, t->data->nTax, 0, t->precision));
     mix(tp.layoutGen);
     mix(t->root);
@@ -917,13 +931,13 @@ static bool buildProgram(Tree *t, int pNum, bool full, int *nOpsOut, int *nKidsO
         if (op.dst >= 0) tp.progSlots.push_back(op.dst);
     bool ok;
     tp.aaLds = 0;
+    tp.aaHbm = false;
     tp.aaRecOff = -1;
     if (tp.wave) {
         *nOpsOut = (int)ops.size();
         *nKidsOut = (int)kids.size();
         ok = buildWaveProgram(t, pNum, ops, kids);
-    } else if (pruneUsesMfma(tp.dim, tp.K, t->precision) && pruneAaCategoryWaves((int)ops.size()) &&
-               pruneAaLdsSlots(tp.K) > 0) {
+    } else if (tp.mfma) {
         ok = buildAaProgram(t, pNum, ops, kids, nOpsOut, nKidsOut);
     } else {
         ok = buildGroupedProgram(t, pNum, ops, kids, nOpsOut, nKidsOut);
@@ -997,42 +1011,11 @@ static bool sethiUllmanOrder(const std::vector<OpRec> &ops, const std::vector<Ki
     return true;
 }
 
-// Fused op records of a 20-state program (AaRec), appended after its kid
-// records: the category kernel reads one per op.
-static bool appendAaRecs(TreePart &tp, const std::vector<OpRec> &ops2, const std::vector<KidRec> &kids2,
-                         size_t *words)
-{
-    const size_t need = *words + ops2.size() * AA_REC_WORDS;
-    if ((int)need > tp.progCapWords) {
-        setError("internal: node program larger than its staging area");
-        return false;
-    }
-    int *r = tp.hProg + *words;
-    for (size_t i = 0; i < ops2.size(); i++, r += AA_REC_WORDS) {
-        const OpRec &o = ops2[i];
-        std::memset(r, 0, sizeof(int) * AA_REC_WORDS);
-        r[0] = o.dst;
-        r[1] = o.flags;
-        r[2] = o.nKids;
-        r[3] = o.kidStart;
-        for (int c = 0; c < 2 && c < o.nKids; c++) {
-            const KidRec &k = kids2[o.kidStart + c];
-            r[4 + 4 * c] = k.kind;
-            r[5 + 4 * c] = k.idx;
-            r[6 + 4 * c] = k.pnode;
-            r[7 + 4 * c] = k.pad;
-        }
-    }
-    tp.aaRecOff = (int)*words;
-    *words = need;
-    return true;
-}
-
-// The 20-state category kernel's program: the ops in Sethi-Ullman order,
-// one group each; a result whose parent is in the program also goes to an
-// LDS slot (op flags bits 8.. = slot + 1), which the parent reads as kid
-// kind 2 (KidRec.pad = the slot; idx still names the partials slot).
-// Results that find no free slot are read back from HBM.
+// The 20-state kernel's program: the ops in Sethi-Ullman order; a result
+// whose parent is in the program also goes to an LDS slot, which the parent
+// reads as child kind 2.  Results that find no free slot are
+// read back from HBM (kind 3).  Staged as the child records, then one AaRec
+// per op.
 static bool buildAaProgram(Tree *t, int pNum, const std::vector<OpRec> &ops, const std::vector<KidRec> &kids,
                            int *nOpsOut, int *nKidsOut)
 {
@@ -1041,7 +1024,7 @@ static bool buildAaProgram(Tree *t, int pNum, const std::vector<OpRec> &ops, con
     std::vector<int> order, parentOp;
     std::vector<std::vector<int>> progKids;
     if (!sethiUllmanOrder(ops, kids, tp.nSlots, order, parentOp, progKids)) return false;
-    const int maxSlots = pruneAaLdsSlots(tp.K);
+    const int maxSlots = pruneAaLdsSlots(tp.K, t->precision);
     std::vector<int> ldsOf(nOps, -1), freeList;
     for (int sl = maxSlots - 1; sl >= 0; sl--) freeList.push_back(sl);
     int used = 0, peak = 0;
@@ -1061,43 +1044,62 @@ static bool buildAaProgram(Tree *t, int pNum, const std::vector<OpRec> &ops, con
     std::vector<int> opOfSlot(tp.nSlots, -1);
     for (int i = 0; i < nOps; i++)
         if (!(ops[i].flags & OP_ROOT)) opOfSlot[ops[i].dst] = i;
-    std::vector<GroupRec> groups;
-    std::vector<OpRec> ops2;
-    std::vector<KidRec> kids2;
-    for (int i : order) {
-        groups.push_back(GroupRec{1, 1, (int)ops2.size(), 0});
-        OpRec o = ops[i];
-        o.flags = (o.flags & 0xff) | ((ldsOf[i] + 1) << 8);
-        o.kidStart = (int)kids2.size();
-        for (int c = 0; c < ops[i].nKids; c++) {
-            KidRec k = kids[ops[i].kidStart + c];
-            if (k.kind == 1) {
-                const int j = opOfSlot[k.idx];
-                if (j >= 0 && parentOp[j] == i && ldsOf[j] >= 0) {
-                    k.kind = 2;
-                    k.pad = ldsOf[j];
-                }
-            }
-            kids2.push_back(k);
-        }
-        ops2.push_back(o);
-    }
-    const size_t words = groups.size() * 4 + ops2.size() * 4 + kids2.size() * 4;
+    const size_t words = ((kids.size() * 4 + 7) & ~(size_t)7) + ops.size() * AA_REC_WORDS;
     if ((int)words > tp.progCapWords) {
         setError("internal: node program larger than its staging area");
         return false;
     }
-    std::memcpy(tp.hProg, groups.data(), groups.size() * sizeof(GroupRec));
-    std::memcpy(tp.hProg + groups.size() * 4, ops2.data(), ops2.size() * sizeof(OpRec));
-    std::memcpy(tp.hProg + (groups.size() + ops2.size()) * 4, kids2.data(), kids2.size() * sizeof(KidRec));
-    size_t allWords = words;
-    if (!appendAaRecs(tp, ops2, kids2, &allWords)) return false;
-    tp.nGroups = (int)groups.size();
-    tp.nKids = (int)kids2.size();
-    tp.progWords = (int)allWords;
+    KidRec *kr = reinterpret_cast<KidRec *>(tp.hProg);
+    int *r = tp.hProg + ((kids.size() * 4 + 7) & ~(size_t)7);
+    int nK = 0;
+    tp.aaHbm = false;
+    const bool f32 = t->precision == FP32;
+    const unsigned matUnits = (unsigned)((size_t)tp.K * aaMatStride(f32) * (f32 ? 4 : 8) / 64);
+    const unsigned slotUnits = (unsigned)(tp.clBytes >> AA_SLOT_SHIFT);
+    const int ldsBytes = aaPartBytes(f32);
+    for (int i : order) {
+        const OpRec &o = ops[i];
+        AaRec rec{};
+        rec.dst = o.dst >= 0 ? (unsigned)o.dst * slotUnits : 0u;
+        rec.ld = ldsOf[i] >= 0 ? ldsOf[i] * ldsBytes : -1;
+        rec.kidStart = nK;
+        for (int c = 0; c < o.nKids; c++) {
+            KidRec k = kids[o.kidStart + c];
+            if (k.kind == 1) {
+                const int j = opOfSlot[k.idx];
+                if (j >= 0 && parentOp[j] == i && ldsOf[j] >= 0) {
+                    k.kind = 2;
+                    k.idx = ldsOf[j] * ldsBytes;
+                } else {
+                    k.kind = j < 0 ? 1 : 3;
+                    k.idx = (int)((unsigned)k.idx * slotUnits);
+                    tp.aaHbm |= j < 0;
+                }
+            }
+            kr[nK++] = k;
+        }
+        KidRec k0 = kr[rec.kidStart], k1 = kr[rec.kidStart + (o.nKids > 1 ? 1 : 0)];
+        if (o.nKids == 2 && k1.kind == 0) std::swap(k0, k1);   // a tip first
+        int type = AA_GEN;
+        if (o.nKids == 2 && !(o.flags & OP_ROOT)) {
+            if (k0.kind == 0) type = k1.kind == 0 ? AA_TT : k1.kind == 2 ? AA_TL : AA_GEN;
+            else if (k0.kind == 2 && k1.kind == 2) type = AA_LL;
+        }
+        rec.info = type | (k0.kind << 2) | (k1.kind << 4) | (o.nKids << 6);
+        rec.mat0 = (unsigned)k0.pnode * matUnits;
+        rec.arg0 = k0.idx;
+        rec.mat1 = (unsigned)k1.pnode * matUnits;
+        rec.arg1 = k1.idx;
+        std::memcpy(r, &rec, sizeof rec);
+        r += AA_REC_WORDS;
+    }
+    tp.nGroups = 0;
+    tp.nKids = nK;
+    tp.aaRecOff = (nK * 4 + 7) & ~7;   // 32-byte aligned
+    tp.progWords = (int)words;
     tp.aaLds = peak;
-    *nOpsOut = (int)ops2.size();
-    *nKidsOut = (int)kids2.size();
+    *nOpsOut = nOps;
+    *nKidsOut = nK;
     return true;
 }
 
@@ -1154,11 +1156,9 @@ static bool buildGroupedProgram(Tree *t, int pNum, const std::vector<OpRec> &ops
     std::memcpy(tp.hProg, groups.data(), groups.size() * sizeof(GroupRec));
     std::memcpy(tp.hProg + groups.size() * 4, ops2.data(), ops2.size() * sizeof(OpRec));
     std::memcpy(tp.hProg + (groups.size() + ops2.size()) * 4, kids2.data(), kids2.size() * sizeof(KidRec));
-    size_t allWords = words;
-    if (pruneUsesMfma(tp.dim, tp.K, t->precision) && !appendAaRecs(tp, ops2, kids2, &allWords)) return false;
     tp.nGroups = (int)groups.size();
     tp.nKids = (int)kids2.size();
-    tp.progWords = (int)allWords;
+    tp.progWords = (int)words;
     *nOpsOut = (int)ops2.size();
     *nKidsOut = (int)kids2.size();
     return true;
@@ -1540,10 +1540,18 @@ static void fillPruneArgs(Tree *t, int pNum, int nOps, PruneArgs &a, bool siteLi
     a.counter = tp.counter;
     a.result = tp.dResultHost;
     a.patLikes = siteLikes ? tp.patLikes : nullptr;
-    a.nLds = tp.aaLds;   // the 20-state category program's slot file (the wave kernels set theirs below)
     a.nTax = dp->nTax;
-    a.tipLds = pruneAaTipLds(dp->nTax) ? 1 : 0;   // the 20-state category kernel's tip codes in LDS
-    a.aaRec = tp.aaRecOff >= 0 ? prog + tp.aaRecOff : nullptr;
+    a.aaRec = nullptr;
+    a.PA = nullptr;
+    a.aaHbm = 0;
+    if (tp.mfma) {
+        a.kids = reinterpret_cast<const KidRec *>(prog);
+        a.nLds = tp.aaLds;
+        a.tipLds = pruneAaTipLds(dp->nTax) ? 1 : 0;
+        a.aaRec = prog + tp.aaRecOff;
+        a.PA = tp.PA;
+        a.aaHbm = tp.aaHbm ? 1 : 0;
+    }
     if (tp.wave) {
         a.wops = reinterpret_cast<const WaveOp *>(prog);
         a.wkids = reinterpret_cast<const WaveKid *>(prog + 16 * tp.nWOps);
@@ -1629,6 +1637,24 @@ static void finishPart(Tree *t, int pNum, bool siteLikes, double lnL, bool bad)
     (void)bad;
 }
 
+// Workgroups of a part's pruning launch.
+static int partBlocks(const TreePart &tp, int precision)
+{
+    return tp.nPatPad / (tp.wave ? pruneWaveTilePatterns(precision) : tp.mfma ? AA_TILE : pruneBlockPatterns(tp.K));
+}
+
+static int g_aaCat = 1, g_aaCatMinOps = 32;
+
+// What a 20-state part counts against the scratch limit: a workgroup per 64
+// patterns, or per 16 in FP32 programs of g_aaCatMinOps ops or more
+// (p4g_setAaTuning), and the general kernel's workgroups in FP64.  The
+// kernel itself has one per 16 patterns, which the array has room for.
+static int noAllocAaBlocks(const TreePart &tp, int precision, int nOps)
+{
+    if (precision == FP64) return tp.nPatPad / pruneBlockPatterns(tp.K);
+    return tp.nPatPad / (g_aaCat && nOps >= std::max(2, g_aaCatMinOps) ? AA_TILE : 4 * AA_TILE);
+}
+
 // Evaluate pending partials + site sum of one part (one launch).  With
 // `scr` (a device address of the no-allocation scratch array) the pruning
 // kernel's reduction scratch is taken from there, the counter is cleared by
@@ -1646,12 +1672,12 @@ static bool evalPart(Tree *t, int pNum, bool full, bool siteLikes, double *lnL, 
     PruneArgs a{};
     fillPruneArgs(t, pNum, nOps, a, siteLikes || cpoSum);
     hipStream_t s = stream();
-    const int nBlocks = tp.wave ? tp.nPatPad / pruneWaveTilePatterns(t->precision)
-                                : tp.nPatPad / pruneBlockPatternsFor(a.dim, a.K, t->precision, nOps);
+    const int nBlocks = partBlocks(tp, t->precision);
     if (scr) {
         // [counter, 256 B][flags int[nBlocks]][sums double[nBlocks]]
         const size_t offBad = 256, offSums = offBad + (((size_t)nBlocks * sizeof(int) + 255) & ~(size_t)255);
-        const size_t need = offSums + (size_t)nBlocks * sizeof(double);
+        const size_t nLim = tp.mfma ? noAllocAaBlocks(tp, t->precision, nOps) : nBlocks;
+        const size_t need = 256 + ((nLim * sizeof(int) + 255) & ~(size_t)255) + nLim * sizeof(double);
         if (need > NOALLOC_SCRATCH_BYTES) {
             (void)hipStreamSynchronize(s);  // queued P kernels read the staging arena
             setError("treeLogLikeNoAlloc: part " + std::to_string(pNum) + " needs " + std::to_string(need) +
@@ -1675,8 +1701,8 @@ static bool evalPart(Tree *t, int pNum, bool full, bool siteLikes, double *lnL, 
     }
     if (g_timing) (void)hipEventRecord(tp.ev0, s);
     const hipError_t le = tp.wave ? launchPruneWave(a, t->precision, nBlocks, tp.waveLds, s)
-                          : pruneUsesMfma(a.dim, a.K, t->precision) ? launchPruneAa(a, nBlocks, s)
-                                                                    : launchPrune(a, t->precision, nBlocks, s);
+                          : tp.mfma ? launchPruneAa(a, t->precision, nBlocks, s)
+                                    : launchPrune(a, t->precision, nBlocks, s);
     if (!hipOk(le, "launch pruning kernel")) {
         (void)hipStreamSynchronize(s);  // queued P kernels read the staging arena
         return false;
@@ -1842,7 +1868,7 @@ static bool derivPart(Tree *t, int pNum, std::vector<double> &out)
     a.nPat = tp.nPat;
     a.nPatPad = tp.nPatPad;
     a.nOps = nOps;
-    a.waveLayout = tp.wave ? 1 : 0;
+    a.layout = tp.wave ? CL_WAVE : tp.mfma ? CL_TILED : CL_GROUPED;
     a.ops = dOps;
     a.sibs = dSibs;
     a.tips = dp->dev.tips;
@@ -1898,7 +1924,8 @@ void p4g_setPmatRoute(int direct)
 
 void p4g_setAaTuning(int categoryWaves, int minOps)
 {
-    setAaTuning(categoryWaves, minOps);
+    g_aaCat = categoryWaves ? 1 : 0;
+    g_aaCatMinOps = minOps < 0 ? 0 : minOps;
 }
 
 void p4g_setWavePreloadLds(int bytes) { setWavePreloadLds(bytes); }
@@ -2765,8 +2792,16 @@ int p4g_copyBigPDecks(p4g_tree *a, p4g_tree *b, int doAll)
         TreePart &A = a->tp[p], &B = b->tp[p];
         const size_t n = (size_t)a->nNodes * A.K * A.dim * A.dim;
         if (!hipOk(hipMemcpyAsync(B.PT64, A.PT64, n * 8, hipMemcpyDeviceToDevice, s), "copy P") ||
-            !hipOk(hipMemcpyAsync(B.PT32, A.PT32, n * 4, hipMemcpyDeviceToDevice, s), "copy P"))
+            (A.PT32 && B.PT32 && !hipOk(hipMemcpyAsync(B.PT32, A.PT32, n * 4, hipMemcpyDeviceToDevice, s), "copy P")))
             return 1;
+        if (B.PA) {
+            // (a's table may be of the other precision)
+            PmatArgs pa{};
+            pa.PT64 = B.PT64;
+            pa.PA = B.PA;
+            pa.paF32 = b->precision == FP32 ? 1 : 0;
+            if (!hipOk(launchAaOperands(pa, a->nNodes * A.K, s), "copy P operands")) return 1;
+        }
         B.pValid = A.pValid;
     }
     return 0;
@@ -2813,7 +2848,13 @@ int p4g_syncChanged(p4g_tree *a, p4g_tree *b)
         for (int n = 0; n < a->nNodes; n++) {
             if (!all && !A.chP[n] && !B.chP[n]) continue;
             r.push_back({A.PT64 + (size_t)n * pe, B.PT64 + (size_t)n * pe, pe * 8});
-            r.push_back({A.PT32 + (size_t)n * pe, B.PT32 + (size_t)n * pe, pe * 4});
+            if (A.PA) {
+                const bool f32 = a->precision == FP32;
+                const size_t pb = (size_t)A.K * aaMatStride(f32) * (f32 ? 4 : 8);
+                r.push_back({(const char *)A.PA + n * pb, (char *)B.PA + n * pb, pb});
+            } else {
+                r.push_back({A.PT32 + (size_t)n * pe, B.PT32 + (size_t)n * pe, pe * 4});
+            }
         }
     }
     if (!r.empty()) {
@@ -2918,14 +2959,17 @@ int p4g_verifyIdentityOfTwoTrees(p4g_tree *a, p4g_tree *b)
         if (!hipOk(hipMemcpy(ca.data(), A.cl, nb, hipMemcpyDeviceToHost), "copy partials") ||
             !hipOk(hipMemcpy(cb.data(), B.cl, nb, hipMemcpyDeviceToHost), "copy partials"))
             return 1;
-        const size_t per = (size_t)A.nPatPad * A.K * A.dim;
+        const size_t per = A.clBytes / (a->precision == FP32 ? 4 : 8);
+        // (20-state FP32 tiles end with their exponents, which are not partials)
+        const size_t tileWords = A.mfma && a->precision == FP32 ? (size_t)A.K * aaPartBytes(true) / 4 : per;
+        const size_t tileVals = A.mfma && a->precision == FP32 ? (size_t)A.K * AA_PART : per;
         for (int node = 0; node < a->nNodes; node++) {
             const int sl = a->slotOf[node];
             if (sl < 0 || node == a->root) continue;
             if (a->precision == FP32) {
                 const float *fa = (const float *)ca.data() + per * sl, *fb = (const float *)cb.data() + per * sl;
                 for (size_t i = 0; i < per; i++)
-                    if (std::fabs((double)fa[i] - (double)fb[i]) > 1e-15) return 1;
+                    if (i % tileWords < tileVals && std::fabs((double)fa[i] - (double)fb[i]) > 1e-15) return 1;
             } else {
                 const double *da = (const double *)ca.data() + per * sl, *db = (const double *)cb.data() + per * sl;
                 for (size_t i = 0; i < per; i++)
@@ -2970,29 +3014,34 @@ int p4g_getCondLikes(const p4g_node *n, int pNum, double *out)
         return 1;
     }
     const int K = tp.K, S = tp.dim, nP = tp.nPat;
-    const size_t per = (size_t)tp.nPatPad * K * S;
+    const bool f32 = t->precision == FP32;
     std::vector<int> e;
     if (!hipOk(hipStreamSynchronize(stream()), "sync")) return 1;
-    std::vector<double> v(per);
-    if (t->precision == FP32) {
-        std::vector<float> f(per);
-        e.resize(tp.sclPerSlot);
-        if (!hipOk(hipMemcpy(f.data(), (const char *)tp.cl + tp.clBytes * sl, per * 4, hipMemcpyDeviceToHost), "copy") ||
-            !hipOk(hipMemcpy(e.data(), tp.scl + (size_t)sl * tp.sclPerSlot, e.size() * 4, hipMemcpyDeviceToHost), "copy"))
-            return 1;
-        for (size_t i = 0; i < per; i++) v[i] = f[i];
-    } else if (!hipOk(hipMemcpy(v.data(), (const char *)tp.cl + tp.clBytes * sl, per * 8, hipMemcpyDeviceToHost), "copy"))
+    std::vector<char> raw(tp.clBytes);
+    if (!hipOk(hipMemcpy(raw.data(), (const char *)tp.cl + tp.clBytes * sl, raw.size(), hipMemcpyDeviceToHost), "copy"))
         return 1;
-    const bool tiled = pruneUsesMfma(S, K, t->precision);
+    if (f32 && !tp.mfma) {
+        e.resize(tp.sclPerSlot);
+        if (!hipOk(hipMemcpy(e.data(), tp.scl + (size_t)sl * tp.sclPerSlot, e.size() * 4, hipMemcpyDeviceToHost), "copy"))
+            return 1;
+    }
+    auto value = [&](size_t i) -> double {
+        return f32 ? (double)reinterpret_cast<const float *>(raw.data())[i] : reinterpret_cast<const double *>(raw.data())[i];
+    };
+    const size_t tileElems = (size_t)K * aaPartBytes(f32) / (f32 ? 4 : 8);   // 20-state tiles: values, then exponents
     for (int k = 0; k < K; k++)
         for (int s = 0; s < S; s++)
             for (int p = 0; p < nP; p++) {
-                // wave layout [k][p][s]; tile-blocked layout of the MFMA
-                // kernel [tile][k][s/4][s%4][p%16]; else [p][k][s]
-                double x = tp.wave ? v[((size_t)k * tp.nPatPad + p) * S + s]
-                           : tiled ? v[(size_t)(p / 16) * K * S * 16 + ((size_t)(k * 5 + s / 4) * 4 + s % 4) * 16 + p % 16]
-                                   : v[((size_t)p * K + k) * S + s];
+                // wave layout [k][p][s]; 20-state tiles [tile][k][aaIndex];
+                // else [p][k][s]
+                const size_t tile = (size_t)(p / AA_TILE) * tileElems;
+                double x = value(tp.wave   ? ((size_t)k * tp.nPatPad + p) * S + s
+                                 : tp.mfma ? tile + (size_t)k * AA_PART + aaIndex(s, p % AA_TILE, f32)
+                                           : ((size_t)p * K + k) * S + s);
                 if (!e.empty()) x = std::ldexp(x, -e[tp.wave ? (size_t)k * tp.nPatPad + p : (size_t)p]);
+                if (f32 && tp.mfma)
+                    x = std::ldexp(x, -reinterpret_cast<const int *>(raw.data())[tile + (size_t)K * AA_PART + k * AA_TILE +
+                                                                               p % AA_TILE]);
                 out[((size_t)k * S + s) * nP + p] = x;
             }
     return 0;
@@ -3224,7 +3273,7 @@ static bool ancLaunch(Tree *t, int pNum, int first, int n, const double *u, uint
     a.dim = tp.dim;
     a.K = tp.K;
     a.nPatPad = tp.nPatPad;
-    a.layout = tp.wave ? CL_WAVE : pruneUsesMfma(tp.dim, tp.K, t->precision) ? CL_TILED : CL_GROUPED;
+    a.layout = tp.wave ? CL_WAVE : tp.mfma ? CL_TILED : CL_GROUPED;
     a.fp32 = t->precision == FP32 ? 1 : 0;
     a.cl = tp.cl;
     a.slotBytes = tp.clBytes;
@@ -3721,12 +3770,7 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
     }
     const int nItems = (int)items.size();
     int nBlocksTot = 0;
-    auto itemBlocks = [](const Item &it) {
-        const ModelPart *mp = it.t->model->parts[it.p];
-        const TreePart &tp = it.t->tp[it.p];
-        return tp.wave ? tp.nPatPad / pruneWaveTilePatterns(it.t->precision)
-                       : tp.nPatPad / pruneBlockPatternsFor(mp->dim, mp->nCat, it.t->precision, it.nOps);
-    };
+    auto itemBlocks = [](const Item &it) { return partBlocks(it.t->tp[it.p], it.t->precision); };
     for (auto &it : items) nBlocksTot += itemBlocks(it);
     if (nItems > b->capItems) {
         devFree(b->dArgs);
@@ -3752,13 +3796,11 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
     auto key = [&](int i) {
         const ModelPart *mp = items[i].t->model->parts[items[i].p];
         const int prec = items[i].t->precision;
-        // MFMA kernels: one launch per (category count, kernel choice) (the
-        // category-split kernel's workgroup is 64 * K threads)
-        const int kc = pruneUsesMfma(mp->dim, mp->nCat, prec)
-                           ? 2 * mp->nCat + (pruneAaCategoryWaves(items[i].nOps) ? 1 : 0)
-                           : 0;
-        // the wave kernel's workgroup size is 64 * K: one launch per K
+        // the 20-state kernel: one launch per (category count, children in
+        // HBM or not), its workgroup is 64 * K threads
         const TreePart &tq = items[i].t->tp[items[i].p];
+        const int kc = tq.mfma ? 2 * mp->nCat + (tq.aaHbm ? 1 : 0) : 0;
+        // the wave kernel's workgroup size is 64 * K: one launch per K
         const int wk = tq.wave ? 16 * tq.nStream + mp->nCat : 0;
         return ((mp->dim * 2 + prec) * 64 + kc) * 32 + wk;
     };
@@ -3778,7 +3820,7 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
     std::vector<std::pair<int, int>> launches;  // (first block, count) per group
     std::vector<int> groupDim, groupPrec;
     std::vector<size_t> groupLds;
-    std::vector<int> groupK, groupWave, groupStreams, groupAaCat, groupAaTip;
+    std::vector<int> groupK, groupWave, groupStreams, groupAa, groupAaHbm, groupAaTip;
     std::vector<size_t> groupAaLds;
     while (j < nItems) {
         const int k0 = key(order[j]);
@@ -3798,19 +3840,19 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
         groupDim.push_back(items[order[j]].t->model->parts[items[order[j]].p]->dim);
         groupPrec.push_back(items[order[j]].t->precision);
         groupK.push_back(items[order[j]].t->model->parts[items[order[j]].p]->nCat);
-        groupAaCat.push_back(pruneAaCategoryWaves(items[order[j]].nOps) ? 1 : 0);
+        groupAa.push_back(items[order[j]].t->tp[items[order[j]].p].mfma ? 1 : 0);
+        groupAaHbm.push_back(b->hArgs[j].aaHbm);
         {
-            // the largest slot file and tip codes of the launch's 20-state category items
+            // the largest slot file and tip codes of the launch's 20-state items
             size_t nl = 0;
             int allTip = 1;
-            const bool aaCat = groupAaCat.back() && pruneUsesMfma(groupDim.back(), groupK.back(), groupPrec.back());
-            for (int q = j; q < jj && aaCat; q++) {
+            for (int q = j; q < jj && groupAa.back(); q++) {
                 const PruneArgs &pa = b->hArgs[q];
-                if (!pruneAaCatItemOk(pa)) {
-                    setError("batch: bad 20-state category program");
+                if (!pruneAaItemOk(pa, groupPrec.back())) {
+                    setError("batch: bad 20-state program");
                     return failQueued();
                 }
-                nl = std::max(nl, pruneAaLdsBytes(pa.K, pa.nLds, pa.tipLds ? pa.nTax : 0));
+                nl = std::max(nl, pruneAaLdsBytes(pa.K, pa.nLds, pa.tipLds ? pa.nTax : 0, groupPrec.back()));
                 allTip &= pa.tipLds ? 1 : 0;
             }
             groupAaLds.push_back(nl);
@@ -3853,9 +3895,9 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
         const int *bi = b->dBlockItem + 2 * launches[g].first;
         const hipError_t le = groupWave[g] ? launchPruneWaveBatch(b->dArgs, bi, launches[g].second, groupK[g],
                                                                  groupStreams[g], groupPrec[g], groupLds[g], s)
-                              : pruneUsesMfma(groupDim[g], groupK[g], groupPrec[g])
-                                  ? launchPruneAaBatch(b->dArgs, bi, launches[g].second, groupK[g], groupAaCat[g] != 0,
-                                                       groupAaLds[g], groupAaTip[g] != 0, s)
+                              : groupAa[g]
+                                  ? launchPruneAaBatch(b->dArgs, bi, launches[g].second, groupK[g], groupPrec[g],
+                                                       groupAaHbm[g] != 0, groupAaLds[g], groupAaTip[g] != 0, s)
                                   : launchPruneBatch(b->dArgs, bi, launches[g].second, groupDim[g], groupPrec[g],
                                                      groupLds[g], s);
         if (!hipOk(le, "launch batched pruning kernel")) return failQueued();

@@ -75,8 +75,11 @@ __global__ __launch_bounds__(64 * DERIV_MAX_K) void k_edgeDerivs(DerivArgs a)
     __shared__ double sL[DERIV_MAX_K][64], sF[DERIV_MAX_K][64], sS[DERIV_MAX_K][64];
     // element (slot, cat, pattern, state) of the down-pass partials
     auto clAt = [&](int slot, int s) -> double {
-        const size_t o = a.waveLayout ? (((size_t)slot * K + cat) * nPP + p) * 4 + s
-                                      : (((size_t)slot * nPP + p) * K + cat) * S + s;
+        const size_t o = a.layout == CL_WAVE ? (((size_t)slot * K + cat) * nPP + p) * 4 + s
+                         : SC == 20 && a.layout == CL_TILED
+                             ? ((size_t)slot * (nPP / AA_TILE) + p / AA_TILE) * K * AA_PART + (size_t)cat * AA_PART +
+                                   aaIndex(s, p % AA_TILE, false)
+                             : (((size_t)slot * nPP + p) * K + cat) * S + s;
         return a.cl[o];
     };
     auto cl2At = [&](int node) -> double * { return a.cl2 + (((size_t)node * K + cat) * nPP + p) * S; };

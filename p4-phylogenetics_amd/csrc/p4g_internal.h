@@ -148,15 +148,61 @@ struct KidRec {
 };
 constexpr int OP_ROOT = 1;
 
-// The 20-state category kernel's fused op record: the op and its first two
-// children in one 64-byte line, [dst, flags, nKids, kidStart, then per
-// child (kind, idx, pnode, pad)], four words spare.  Written after the kid
-// records of that program; the kernel reads it one op ahead.
-constexpr int AA_REC_WORDS = 16;
+// The 20-state kernel's op record, one 32-byte scalar load, written after the
+// kid records of the program.  Child kinds: 0 tip (arg: tip row), 1 partials
+// slot left by an earlier evaluation (arg: its offset, as dst), 2 LDS slot
+// (arg: its byte offset), 3 partials slot written by this program (arg: as
+// 1); mat: the child's matrices in the operand table, in units of 64 bytes
+// (an op with one child repeats it).
+enum { AA_TT = 0, AA_TL = 1, AA_LL = 2, AA_GEN = 3 };
 struct AaRec {
-    int dst, flags, nKids, kidStart;
-    int kind[2], idx[2], pnode[2], slot[2];
+    unsigned dst;   // offset of the result's partials slot in units of 2^AA_SLOT_SHIFT bytes
+    int info;       // type in bits 0..1 (two tips; tip and LDS slot; two LDS slots; any other),
+                    // kinds in bits 2..3 and 4..5, number of children above
+    unsigned mat0;
+    int arg0;
+    unsigned mat1;
+    int arg1;
+    int kidStart;   // its first kid record (children past the second)
+    int ld;         // byte offset of the result's LDS slot, or -1
 };
+static_assert(sizeof(AaRec) == 32, "AaRec is one 32-byte scalar load");
+constexpr int AA_REC_WORDS = 8;
+constexpr int AA_SLOT_SHIFT = 9;   // a slot holds a multiple of 16 tiles
+constexpr int AA_S = 20;
+constexpr int AA_TILE = 16;            // patterns per tile
+constexpr int AA_PART = AA_S * AA_TILE;   // values of one (tile, category)
+// Tile layout of a 20-state partial: [slot][tile]([cat][AA_PART] values, and
+// in FP32 [cat][AA_TILE] scale exponents), the value of state s and pattern
+// p of the tile at aaIndex(s, p): lane l = 16 q + p of the kernel's wave
+// holds states 4q .. 4q+3 and 16 + q, in 16-byte stores of the wave and one
+// scalar store.  The exponents sit with their tile, so one address serves
+// both and a slot is one range to copy.
+constexpr int aaPartBytes(bool fp32) { return fp32 ? AA_PART * 4 + AA_TILE * 4 : AA_PART * 8; }
+__host__ __device__ inline int aaIndex(int s, int p, bool fp32)
+{
+    if (s >= 16) return 256 + (s - 16) * 16 + p;
+    const int V = fp32 ? 4 : 2, r = s & 3, lane = (s >> 2) * 16 + p;
+    return (r / V) * (64 * V) + lane * V + r % V;
+}
+// The operand table of a 20-state part, AA_MAT values per (node, category):
+// P in the order of the matrix instructions' A operands -- k-steps 0..3 of
+// the rows 0..15 by lane, k-step 4, then the same of the rows 16..19.  The
+// FP32 and FP64 instructions order their result rows differently, hence two
+// row orders.
+constexpr int AA_MAT = AA_S * AA_S;
+// The table's stride: whole 128-byte lines, and the operands' parts start on
+// lines, so no two loads of a matrix touch the same line (the L1 stalls on a
+// second access to a line that is still on its way).
+constexpr int aaMatStride(bool fp32) { return fp32 ? 416 : 400; }
+__host__ __device__ inline int aaPaIndex(int s, int j, bool fp32)
+{
+    if (s < 16) {
+        const int row = fp32 ? s : (s & 3) * 4 + (s >> 2);
+        return j < 16 ? ((j >> 2) * 16 + row) * 4 + (j & 3) : 256 + (j - 16) * 16 + row;
+    }
+    return j < 16 ? 320 + ((j >> 2) * 4 + (s - 16)) * 4 + (j & 3) : 384 + (j - 16) * 4 + (s - 16);
+}
 
 // Program of the wave-per-category DNA kernel (k_pruneWave): one 16-int
 // record per node, in execution order, children inline (up to 3; more in
@@ -225,9 +271,13 @@ struct TreePart {
     // P^T per node and category: [nNodes][K][dim(j)][dim(s)] = P[s][j]
     double *PT64 = nullptr;
     float *PT32 = nullptr;
+    // 20-state parts of the matrix-core kernel: its operand table, float or
+    // double by precision ([nNodes][K][AA_MAT]; PT32 is not kept then)
+    void *PA = nullptr;
     // Partials: [nSlots][nPatPad][K][dim] of float or double, scale
     // exponents [nSlots][nPatPad] (FP32 mode); the wave kernel's layout is
-    // [nSlots][K][nPatPad][dim] with exponents [nSlots][K][nPatPad].
+    // [nSlots][K][nPatPad][dim] with exponents [nSlots][K][nPatPad]; the
+    // 20-state kernel's are tiles with their exponents (aaIndex; no scl).
     void *cl = nullptr;
     int *scl = nullptr;
     size_t clBytes = 0;
@@ -246,7 +296,9 @@ struct TreePart {
     int nWOps = 0, nWKids = 0, nPre = 0, nLds = 0, tipLds = 0, nKidTot = 0;
     int nStream = 1, nS0 = 0;
     int popsOff = 0;               // LeanOp records, in ints from the program start
-    int aaLds = 0;                 // LDS slots of the 20-state category program
+    bool mfma = false;             // the 20-state matrix-core kernel
+    int aaLds = 0;                 // LDS slots of the 20-state program
+    bool aaHbm = false;            // it reads partials that earlier evaluations left in HBM
     int aaRecOff = -1;             // word offset of its fused op records in the program, or -1
     int tipPnOff = 0, nTipKid = 0; // staged tip children's P^T nodes
     // The staged program is reused while everything it depends on is
@@ -353,6 +405,8 @@ struct PmatArgs {
     const double *V, *Vi, *lam;
     double *PT64;
     float *PT32;
+    void *PA;               // operand table of the 20-state kernel, or null (PT32 is null with it)
+    int paF32;              // its values are float
 };
 
 struct PruneArgs {
@@ -397,7 +451,9 @@ struct PruneArgs {
     const int *tipPn;
     int nAmb;                // entries of ambMask
     int ptWarmBytes;         // lean kernel: bytes of P^T to pull into L2 at the start (0: none)
-    const int *aaRec;        // 20-state category kernel: fused op records, [nOps][AA_REC_WORDS]
+    const int *aaRec;        // 20-state kernel: fused op records, [nOps][AA_REC_WORDS]
+    const void *PA;          // and its operand table, float or double by precision
+    int aaHbm;
 };
 
 // ---------------------------------------------- branch-length derivatives
@@ -423,7 +479,7 @@ struct DerivPArgs {
 };
 struct DerivArgs {
     int dim, K, nPat, nPatPad, nOps;
-    int waveLayout;              // the down-pass partials are [slot][cat][pattern][4]
+    int layout;                  // of the down-pass partials (CL_*)
     const DerivOp *ops;
     const DerivSib *sibs;
     const uint8_t *tips;
@@ -453,6 +509,8 @@ hipError_t launchPmatMulti(const PmatArgs *args, const int *first, int nItems, i
 // eigIn (4-state parts only); pmatDirect(dim) says whether that route is on.
 hipError_t launchPexp(const PmatArgs &a, const double *eigIn, hipStream_t s);
 bool pmatDirect(int dim);
+// the 20-state kernel's operand table of n matrices from a.PT64
+hipError_t launchAaOperands(const PmatArgs &a, int n, hipStream_t s);
 // Direct P (dim 4 or 20) for several items in one launch: args/ins/first
 // are device-readable arrays of nItems entries (first: nItems + 1 prefix
 // sums of each item's nItems * K matrices, first[nItems] == total).
@@ -461,12 +519,6 @@ hipError_t launchPexpMulti(int dim, const PmatArgs *args, const double *const *i
 // 20-state flushes with fewer pending P matrices use the eigen route.
 constexpr int PEXP_WAVE_MIN_ITEMS = 16;
 void setPmatRoute(int direct);
-// 20-state FP32 pruning: one wavefront per (tile, category) for programs
-// of at least minOps ops when catWaves is on (the default), else one per
-// tile with every category.
-constexpr int AA_CAT_MIN_OPS = 32;
-void setAaTuning(int catWaves, int minOps);
-bool pruneAaCategoryWaves(int nOps);
 hipError_t launchPrune(const PruneArgs &a, int precision, int nBlocks, hipStream_t s);
 hipError_t launchPruneBatch(const PruneArgs *dArgs, const int *dBlockItem, int nBlocks,
                             int dim, int precision, size_t lds, hipStream_t s);
@@ -474,18 +526,18 @@ int pruneBlockPatterns(int K);  // patterns per 256-thread block
 int pruneGroupWidthFor(int dim, int precision);  // ops per binary group
 void setPruneTuning(int precision, int G, int lds);
 size_t pruneLdsBytes(int nKids, int K, int dim, int precision);  // 0 if P stays in global
-// 20-state FP32 parts use the MFMA kernel and a tile-blocked partial layout
+// 20-state parts with at most WAVE_MAX_K categories use the matrix-core
+// kernel (p4g_aa.hip): tiles of AA_TILE patterns, layout aaIndex.
 bool pruneUsesMfma(int dim, int K, int precision);
-int pruneBlockPatternsFor(int dim, int K, int precision, int nOps);
-hipError_t launchPruneAa(const PruneArgs &a, int nBlocks, hipStream_t s);
-hipError_t launchPruneAaBatch(const PruneArgs *d, const int *bi, int nBlocks, int K, bool catWaves, size_t ldsBytes,
-                              bool tipLds, hipStream_t s);
-// the category kernel's LDS slot file: the most slots a program may use
-// (0: none), and the bytes of n slots
-int pruneAaLdsSlots(int K);
-size_t pruneAaLdsBytes(int K, int nLds, int tipTaxa);
+hipError_t launchPruneAa(const PruneArgs &a, int precision, int nBlocks, hipStream_t s);
+hipError_t launchPruneAaBatch(const PruneArgs *d, const int *bi, int nBlocks, int K, int precision, bool hbm,
+                              size_t lds, bool tipLds, hipStream_t s);
+// its LDS slot file: the most slots a program may use (0: none), and the
+// bytes of n slots and the staged tip codes
+int pruneAaLdsSlots(int K, int precision);
+size_t pruneAaLdsBytes(int K, int nLds, int tipTaxa, int precision);
 bool pruneAaTipLds(int nTax);
-bool pruneAaCatItemOk(const PruneArgs &a);
+bool pruneAaItemOk(const PruneArgs &a, int precision);
 void setAaLdsSlots(int n);
 // 4-state parts with at most WAVE_MAX_K categories use the wave-per-category
 // kernel: partials [slot][cat][pattern][state], FP32 exponents
@@ -556,8 +608,7 @@ constexpr int ANC_MAX_K = 16;
 // Where the partials of a slot live (the layouts of the pruning kernels).
 constexpr int CL_GROUPED = 0;   // [slot][pattern][cat][state], exponents [slot][pattern]
 constexpr int CL_WAVE = 1;      // [slot][cat][pattern][4],     exponents [slot][cat][pattern]
-constexpr int CL_TILED = 2;     // 20 states: [slot][pattern/16][cat][state/4][state%4][pattern%16],
-                                // exponents [slot][pattern]
+constexpr int CL_TILED = 2;     // 20 states: tiles of 16 patterns with their exponents (aaIndex)
 struct AncArgs {
     int dim, K, nPatPad, layout, fp32;
     const void *cl;              // the tree part's partials

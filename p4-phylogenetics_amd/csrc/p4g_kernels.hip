@@ -21,6 +21,7 @@
 //           exact power of two when its max over categories and states
 //           drops below 2^-24, accumulating integer exponents per node.
 #include "p4g_internal.h"
+#include "p4g_site.h"
 
 #include <cmath>
 
@@ -209,6 +210,33 @@ hipError_t launchEig(const EigArgs &a, hipStream_t s)
 }
 
 // ------------------------------------------------------------- P matrices
+// P[i][j] into the 20-state kernel's operand table (m: the matrix's first
+// value).
+__device__ __forceinline__ void aaPut(const PmatArgs &a, size_t m, int i, int j, double pij)
+{
+    if (a.paF32)
+        ((float *)a.PA)[m + aaPaIndex(i, j, true)] = (float)pij;
+    else
+        ((double *)a.PA)[m + aaPaIndex(i, j, false)] = pij;
+}
+
+// The operand table of n matrices from their P^T (a copy of P matrices
+// between trees of different precision).
+__global__ __launch_bounds__(256) void k_aaOperands(PmatArgs a, int n)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= n * AA_S * AA_S) return;
+    const int m = e / (AA_S * AA_S), r = e - m * (AA_S * AA_S), j = r / AA_S, i = r - j * AA_S;
+    aaPut(a, (size_t)m * aaMatStride(a.paF32), i, j, a.PT64[e]);
+}
+
+hipError_t launchAaOperands(const PmatArgs &a, int n, hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_aaOperands, dim3(((size_t)n * AA_S * AA_S + 255) / 256), dim3(256), 0, s, a, n);
+    return hipGetLastError();
+}
+
 __device__ __forceinline__ void pmatBody(const PmatArgs &a, long gid)
 {
     const int S = a.dim, K = a.K;
@@ -227,7 +255,10 @@ __device__ __forceinline__ void pmatBody(const PmatArgs &a, long gid)
     const double pij = (i == j ? 1.0 : 0.0) + acc;
     const size_t o = (((size_t)node * K + k) * S + j) * S + i;
     a.PT64[o] = pij;
-    a.PT32[o] = (float)pij;
+    if (a.PA)
+        aaPut(a, ((size_t)node * K + k) * aaMatStride(a.paF32), i, j, pij);
+    else
+        a.PT32[o] = (float)pij;
 }
 
 __global__ __launch_bounds__(256) void k_pmat(PmatArgs a)
@@ -641,7 +672,10 @@ __device__ __forceinline__ void pexpWaveBody(const PmatArgs &a, const double *in
         const int i = e / S, j = e - (e / S) * S;
         const double pij = (i == j ? 1.0 : 0.0) + W[e];
         a.PT64[o + j * S + i] = pij;
-        a.PT32[o + j * S + i] = (float)pij;
+        if (a.PA)
+            aaPut(a, ((size_t)node * a.K + k) * aaMatStride(a.paF32), i, j, pij);
+        else
+            a.PT32[o + j * S + i] = (float)pij;
     }
 }
 
@@ -710,7 +744,6 @@ hipError_t launchPexp(const PmatArgs &a, const double *eigIn, hipStream_t s)
 
 // ----------------------------------------------------------------- pruning
 constexpr int PRUNE_THREADS = 256;
-constexpr float SCALE_THRESH = 5.9604645e-08f;  // 2^-24
 
 int pruneBlockPatterns(int K)
 {
@@ -796,74 +829,6 @@ __device__ __forceinline__ void rescale(T *acc, int &e, int S, int Kp)
             if (s < S) acc[s] = ldexp(acc[s], E);
         e += E;
     }
-}
-
-// Site likelihood of pattern p from the root's category-summed
-// sum_s pi_s cl_s (Lk) and the pattern's scale exponent e, as
-// Pf/p4_tree.c:1029-1197: (1 - pInvar)/K * Lk plus the invariant-site term,
-// or Lk/K without pInvar; adds count * log(like) to contrib.  In FP32 mode
-// the partials carry 2^-e, so the variable-site part is unscaled in FP64
-// before the invariant part is added; with no invariant part the log is
-// taken in the scaled domain.
-template <bool SCALE>
-__device__ __forceinline__ void siteLogLike(const PruneArgs &a, double Lk, int e, int p, int K,
-                                            const double *pi, double &contrib, int &bad)
-{
-    const size_t nPatPad = (size_t)a.nPatPad;
-    const double LN2 = 0.69314718055994530942;
-    double like, lnl;
-    bool ok;
-    if (a.pInvar != 0.0) {
-        const double varS = Lk * ((1.0 - a.pInvar) / (double)K);
-        double inv = 0.0;
-        for (int w = 0; w < a.nWords; w++) {
-            uint32_t mw = a.invMask[(size_t)w * nPatPad + p];
-            while (mw) {
-                const int b = __ffs(mw) - 1;
-                mw &= mw - 1;
-                inv += pi[w * 32 + b] * a.pInvar;
-            }
-        }
-        if (SCALE && e != 0 && inv == 0.0) {
-            ok = varS > 0.0;
-            lnl = log(varS) - (double)e * LN2;
-            like = ldexp(varS, -e);
-        } else {
-            like = ((SCALE && e != 0) ? ldexp(varS, -e) : varS) + inv;
-            ok = like > 0.0;
-            lnl = log(like);
-        }
-    } else {
-        const double likeS = (K > 1) ? Lk / (double)K : Lk;
-        ok = likeS > 0.0;
-        lnl = log(likeS);
-        like = likeS;
-        if (SCALE && e != 0) {
-            lnl -= (double)e * LN2;
-            like = ldexp(likeS, -e);
-        }
-    }
-    if (p < a.nPat) {
-        if (!ok) bad = 1;
-        contrib = a.counts[p] * lnl;
-        if (a.patLikes) a.patLikes[p] = like;
-    }
-}
-
-// A workgroup's sum and flag for the workgroup that will add them all, and
-// its ticket.  The two stores are agent-scope atomics (written through to
-// memory) and acknowledged before the ticket is drawn, which is all the
-// reader's agent-scope loads need.  A release fence in their place writes the
-// XCD's whole L2 back to memory, once per workgroup, with the other
-// workgroups' partials dirty in it: dirty paths of 24 parts x 4 chains took
-// 303 us in the 4-state kernel with it and take 104 us, a 64-taxon,
-// 38,184-pattern FP32 evaluation 88 us and 70.
-__device__ __forceinline__ unsigned postBlockSum(const PruneArgs &a, double contrib, int bad, int blk)
-{
-    __hip_atomic_store(a.blockSums + blk, contrib, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(a.blockBad + blk, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    return __hip_atomic_fetch_add(a.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Workgroup reduction of the per-lane weighted site log likelihoods, then
@@ -1256,719 +1221,6 @@ hipError_t launchPruneBatch(const PruneArgs *dArgs, const int *dBlockItem, int n
     }
 }
 
-// ------------------------------------------------ 20-state pruning on MFMA
-// One wavefront owns a tile of 16 site patterns (all gamma categories); a
-// 256-thread workgroup owns 4 tiles.  Partials of a 20-state FP32 part are
-// tile-blocked, [slot][tile][cat][t = state/4][state%4][pattern%16], so the
-// B operand of v_mfma_f32_16x16x4f32 for k-step t is 64 consecutive floats.
-// Per child and category: out[s][p] = sum_j P[s][j] x[j][p] as 5 k-steps
-// of 4 on two 16-row tiles (states 0-15 and 16-19; rows 20-31 are zero
-// padding), with A[s][j] = P^T[j][s] read from the P^T table.
-// Lane l holds A[l%16][l/16], B[l/16][l%16] and D rows 4*(l/16)+r, r<4,
-// of column l%16.
-typedef float f4v __attribute__((ext_vector_type(4)));
-constexpr int AA_S = 20;
-constexpr int AA_TILE = 16;
-
-__device__ __forceinline__ f4v mfma4(float a, float b, f4v c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-template <int KC>
-__device__ __forceinline__ void pruneAaBody(const PruneArgs &a, int blk, int nBlk)
-{
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int q = lane >> 4, pl = lane & 15;
-    const int K = a.K;
-    const int tile = blk * (PRUNE_THREADS / 64) + wave;
-    const int p = tile * AA_TILE + pl;
-    const size_t nPatPad = (size_t)a.nPatPad;
-    const size_t tileFloats = (size_t)K * AA_S * AA_TILE;
-    const size_t slotFloats = nPatPad * K * AA_S;
-    const float *PT = (const float *)a.PT;
-    float *cl = (float *)a.cl;
-    const f4v zero = {0.f, 0.f, 0.f, 0.f};
-    const f4v ones = {1.f, 1.f, 1.f, 1.f};
-
-    double contrib = 0.0;
-    int bad = 0;
-    for (int g = 0; g < a.nGroups; ++g) {
-        const GroupRec gr = a.groups[g];
-        for (int o = 0; o < gr.nOps; ++o) {
-            const OpRec op = a.ops[gr.opStart + o];
-            f4v pr0[KC], pr1[KC];
-            int e = 0;
-            for (int c = 0; c < op.nKids; ++c) {
-                const KidRec kd = a.kids[op.kidStart + c];
-                const float *Pn = PT + (size_t)kd.pnode * K * AA_S * AA_S;
-                f4v v0[KC], v1[KC];
-                bool skip = false;
-                if (kd.kind == 0) {
-                    const unsigned code = a.tips[(size_t)kd.idx * nPatPad + p];
-                    skip = (code == TIP_ALL) && c != 0;
-#pragma unroll
-                    for (int k = 0; k < KC; k++) {
-                        if (k >= K) break;
-                        const float *Pk = Pn + k * AA_S * AA_S;
-                        if (code < (unsigned)AA_S) {
-                            v0[k] = *reinterpret_cast<const f4v *>(Pk + code * AA_S + 4 * q);
-                            v1[k] = q == 0 ? *reinterpret_cast<const f4v *>(Pk + code * AA_S + 16) : zero;
-                        } else if (code == TIP_ALL) {
-                            v0[k] = ones;
-                            v1[k] = q == 0 ? ones : zero;
-                        } else {
-                            const uint64_t m = a.ambMask[code - AA_S];
-                            v0[k] = zero;
-                            v1[k] = zero;
-                            for (int j = 0; j < AA_S; j++)
-                                if ((m >> j) & 1ull) {
-                                    v0[k] += *reinterpret_cast<const f4v *>(Pk + j * AA_S + 4 * q);
-                                    if (q == 0) v1[k] += *reinterpret_cast<const f4v *>(Pk + j * AA_S + 16);
-                                }
-                        }
-                    }
-                } else {
-                    const float *X = cl + (size_t)kd.idx * slotFloats + (size_t)tile * tileFloats;
-#pragma unroll
-                    for (int k = 0; k < KC; k++) {
-                        if (k >= K) break;
-                        const float *Pk = Pn + k * AA_S * AA_S;
-                        f4v acc0 = zero, acc1 = zero;
-#pragma unroll
-                        for (int t = 0; t < 5; t++) {
-                            const float b = X[(k * 5 + t) * 64 + lane];
-                            const float a0 = Pk[(4 * t + q) * AA_S + pl];
-                            const float a1 = pl < 4 ? Pk[(4 * t + q) * AA_S + 16 + pl] : 0.f;
-                            acc0 = mfma4(a0, b, acc0);
-                            acc1 = mfma4(a1, b, acc1);
-                        }
-                        v0[k] = acc0;
-                        v1[k] = acc1;
-                    }
-                    e += a.scl[(size_t)kd.idx * nPatPad + p];
-                }
-#pragma unroll
-                for (int k = 0; k < KC; k++) {
-                    if (k >= K) break;
-                    if (c == 0) {
-                        pr0[k] = v0[k];
-                        pr1[k] = v1[k];
-                    } else if (!skip) {
-                        pr0[k] *= v0[k];
-                        pr1[k] *= v1[k];
-                    }
-                }
-            }
-            // rescale: max over categories and states of this pattern
-            float m = 0.f;
-#pragma unroll
-            for (int k = 0; k < KC; k++) {
-                if (k >= K) break;
-                for (int r = 0; r < 4; r++) m = fmaxf(m, fmaxf(pr0[k][r], pr1[k][r]));
-            }
-            m = fmaxf(m, __shfl_xor(m, 16));
-            m = fmaxf(m, __shfl_xor(m, 32));
-            if (m < SCALE_THRESH && m > 0.f) {
-                int ex;
-                frexpf(m, &ex);
-                const int E = -ex;
-#pragma unroll
-                for (int k = 0; k < KC; k++) {
-                    if (k >= K) break;
-                    for (int r = 0; r < 4; r++) {
-                        pr0[k][r] = ldexpf(pr0[k][r], E);
-                        pr1[k][r] = ldexpf(pr1[k][r], E);
-                    }
-                }
-                e += E;
-            }
-            if (!(op.flags & OP_ROOT)) {
-                float *D = cl + (size_t)op.dst * slotFloats + (size_t)tile * tileFloats;
-#pragma unroll
-                for (int k = 0; k < KC; k++) {
-                    if (k >= K) break;
-                    for (int r = 0; r < 4; r++) D[((k * 5 + q) * 4 + r) * AA_TILE + pl] = pr0[k][r];
-                    if (q == 0)
-                        for (int r = 0; r < 4; r++) D[((k * 5 + 4) * 4 + r) * AA_TILE + pl] = pr1[k][r];
-                }
-                if (q == 0) a.scl[(size_t)op.dst * nPatPad + p] = e;
-                continue;
-            }
-            // root: sum_k sum_s pi_s cl_s over this lane's states, then
-            // across the four lanes of the pattern
-            const double *pi = a.rootPi;
-            uint64_t msk = ~0ull;
-            if (a.rootLeafRow >= 0) {
-                const unsigned code = a.tips[(size_t)a.rootLeafRow * nPatPad + p];
-                msk = code < (unsigned)AA_S ? (1ull << code) : code == TIP_ALL ? ~0ull : a.ambMask[code - AA_S];
-            }
-            double Lk = 0.0;
-#pragma unroll
-            for (int k = 0; k < KC; k++) {
-                if (k >= K) break;
-                for (int r = 0; r < 4; r++) {
-                    const int s0 = 4 * q + r;
-                    if ((msk >> s0) & 1ull) Lk += pi[s0] * (double)pr0[k][r];
-                    if (q == 0 && ((msk >> (16 + r)) & 1ull)) Lk += pi[16 + r] * (double)pr1[k][r];
-                }
-            }
-            Lk += __shfl_xor(Lk, 16);
-            Lk += __shfl_xor(Lk, 32);
-            if (q == 0) siteLogLike<true>(a, Lk, e, p, K, pi, contrib, bad);
-        }
-    }
-    finishSiteSum(a, contrib, bad, blk, nBlk);
-}
-
-template <int KC>
-__global__ __launch_bounds__(PRUNE_THREADS) void k_pruneAa(PruneArgs a)
-{
-    pruneAaBody<KC>(a, blockIdx.x, gridDim.x);
-}
-
-__device__ __forceinline__ void finishSiteSumWave(const PruneArgs &a, double contrib, int bad, int blk, int nBlk);
-
-// Category-split variant: one wavefront per (16-pattern tile, category),
-// the K category waves of a tile in one workgroup, so a launch has K times
-// the wavefronts and each walks the program with a K-th of the work.  The
-// scale exponent stays per (node, pattern): every wave posts its
-// per-pattern maximum in LDS (double-buffered, one barrier per op) and all
-// take the maximum over categories, so partials and exponents are those of
-// k_pruneAa bit for bit; only the FP64 root sum over categories is added
-// in another order.
-//
-// Children computed earlier in the same launch come from an LDS slot file
-// (a.nLds slots; op flags bits 8.. = the result's slot + 1, kid kind 2 =
-// read slot KidRec.pad): per slot and category wave the tile's 20 x 16
-// values in the global tile layout, and the wave's own copy of the 16
-// exponents (every wave computes the same exponents, so no wave reads
-// another's).  Only the wave that wrote a slot region reads it, in program
-// order, so no barrier is needed for it.  With a.tipLds the tile's tip
-// codes ([nTax][16] bytes) are staged in LDS once.
-//
-// Stores are deferred by one op.  The vector memory counter retires loads
-// and stores in issue order, so a load issued after an op's HBM stores
-// waits for their acknowledgement as well.  Here the P rows (and tip rows)
-// of an op's first two children, which depend on the program only, are
-// loaded while the op before it finishes; the op then issues the previous
-// op's HBM stores (from LDS, where each result is staged), reads its
-// children's partials (LDS, or HBM after those stores) and computes, so no
-// load queues behind a store.  Every wave writes the (identical) exponents
-// of a result, so a later op reads exponents its own wave wrote.
-template <bool TIPLDS>
-__device__ __forceinline__ void pruneAaCatBody(const PruneArgs &a, int tile, int nTiles)
-{
-    __shared__ float mx[2][WAVE_MAX_K][AA_TILE];
-    __shared__ double rootL[WAVE_MAX_K][AA_TILE];
-    __shared__ int rootE[AA_TILE];
-    // [nLds + 1][K][320] values, [nLds + 1][K][16] exponents (region nLds:
-    // the staged result of an op without a slot), [nTax][16] tip codes
-    extern __shared__ float aaSlots[];
-    const int tid = threadIdx.x;
-    const int k = __builtin_amdgcn_readfirstlane(tid >> 6);   // category
-    const int lane = tid & 63;
-    const int q = lane >> 4, pl = lane & 15;
-    const int K = a.K;
-    const int p = tile * AA_TILE + pl;
-    const size_t nPatPad = (size_t)a.nPatPad;
-    const size_t tileFloats = (size_t)K * AA_S * AA_TILE;
-    const size_t slotFloats = nPatPad * K * AA_S;
-    const float *PT = (const float *)a.PT;
-    float *cl = (float *)a.cl;
-    const f4v zero = {0.f, 0.f, 0.f, 0.f};
-    const f4v ones = {1.f, 1.f, 1.f, 1.f};
-
-    int *slotEx = reinterpret_cast<int *>(aaSlots + (size_t)(a.nLds + 1) * K * 320);
-    uint8_t *tipL = reinterpret_cast<uint8_t *>(slotEx + (size_t)(a.nLds + 1) * K * AA_TILE);
-    if (TIPLDS) {
-        for (int t = tid; t < a.nTax; t += blockDim.x)
-            *reinterpret_cast<uint4 *>(tipL + t * AA_TILE) =
-                *reinterpret_cast<const uint4 *>(a.tips + (size_t)t * nPatPad + (size_t)tile * AA_TILE);
-        __syncthreads();
-    }
-    // (two separate loads, not a select of pointers: a generic pointer
-    // would make every tip code a flat load waiting on both counters)
-    auto tipCode = [&](int row) -> unsigned {
-        if (TIPLDS) return (unsigned)tipL[row * AA_TILE + pl];
-        return (unsigned)a.tips[(size_t)row * nPatPad + p];
-    };
-    // a tip row of P: this lane's four states, and states 16..19 (used on
-    // q == 0 only; pr1 of the other lanes is cleared before it is used)
-    auto tipRow = [&](const float *Pk, unsigned code, f4v &v0, f4v &v1) {
-        if (code < (unsigned)AA_S) {
-            v0 = *reinterpret_cast<const f4v *>(Pk + code * AA_S + 4 * q);
-            v1 = *reinterpret_cast<const f4v *>(Pk + code * AA_S + 16);
-        } else if (code == TIP_ALL) {
-            v0 = ones;
-            v1 = ones;
-        } else {
-            const uint64_t m = a.ambMask[code - AA_S];
-            v0 = zero;
-            v1 = zero;
-            for (int j = 0; j < AA_S; j++)
-                if ((m >> j) & 1ull) {
-                    v0 += *reinterpret_cast<const f4v *>(Pk + j * AA_S + 4 * q);
-                    v1 += *reinterpret_cast<const f4v *>(Pk + j * AA_S + 16);
-                }
-        }
-    };
-    // The pending result: an op leaves its values and exponents in LDS (its
-    // slot, or region nLds) and the next op copies them to HBM after its
-    // own loads, so nothing of it occupies registers meanwhile.  Addresses
-    // are a wave-uniform base plus a 32-bit unsigned lane byte offset (the
-    // scalar-base + vector-offset form of the global instructions).
-    bool pend = false;
-    int pDst = 0, pSrc = 0;
-    const unsigned laneB = (unsigned)(q * 64 + pl) * 4u;   // state 4q, pattern pl of a [20][16] tile
-    const unsigned laneW = (unsigned)lane * 4u;            // state q (of four), pattern pl
-    const unsigned plB = (unsigned)pl * 4u;
-    // Every lane stores the same number of words (no branch on q): states
-    // 0..15 in four stores, states 16 + q in one, and the pattern's
-    // exponent (four lanes write each, the same value).  The stores are
-    // non-temporal: the launch's partials stream through L2 once, and
-    // would otherwise evict the P matrices every op gathers from there.
-    auto flush = [&]() {
-        const float *L = aaSlots + ((size_t)pSrc * K + k) * 320;
-        char *D = (char *)(cl + (size_t)pDst * slotFloats + (size_t)tile * tileFloats + (size_t)k * 320);
-        float v[5];
-        for (int r = 0; r < 4; r++) v[r] = L[(q * 4 + r) * AA_TILE + pl];
-        v[4] = L[256 + q * AA_TILE + pl];
-        const int ex = slotEx[((size_t)pSrc * K + k) * AA_TILE + pl];
-        for (int r = 0; r < 4; r++) __builtin_nontemporal_store(v[r], (float *)(D + 64 * r + laneB));
-        __builtin_nontemporal_store(v[4], (float *)(D + 1024 + laneW));
-        __builtin_nontemporal_store(ex, (int *)((char *)(a.scl + (size_t)pDst * nPatPad + (size_t)tile * AA_TILE) + plB));
-        pend = false;
-    };
-
-    // The program: op i's fused record (AaRec, 16 words) is loaded one op
-    // ahead, lanes 0..11 one word each (a single vector load into one
-    // register), and taken apart with readlane when the op before it
-    // finishes: a scalar load there would wait out a scalar-cache miss on
-    // most ops.  Children past the second (a root with three or more) come
-    // from the kid records.
-    typedef int i4v __attribute__((ext_vector_type(4)));
-    typedef const __attribute__((address_space(4))) i4v ci4v;
-    ci4v *kidsC = (ci4v *)a.kids;
-    auto kidAt = [&](int i) -> KidRec {
-        const i4v r = kidsC[i];
-        return KidRec{r.x, r.y, r.z, r.w};
-    };
-    const int *recG = a.aaRec;
-    auto recLoad = [&](int i) -> int { return lane < 12 ? recG[(size_t)i * AA_REC_WORDS + lane] : 0; };
-    auto recTake = [&](int v) -> AaRec {
-        AaRec r;
-        r.dst = __builtin_amdgcn_readlane(v, 0);
-        r.flags = __builtin_amdgcn_readlane(v, 1);
-        r.nKids = __builtin_amdgcn_readlane(v, 2);
-        r.kidStart = __builtin_amdgcn_readlane(v, 3);
-        for (int c = 0; c < 2; c++) {
-            r.kind[c] = __builtin_amdgcn_readlane(v, 4 + 4 * c);
-            r.idx[c] = __builtin_amdgcn_readlane(v, 5 + 4 * c);
-            r.pnode[c] = __builtin_amdgcn_readlane(v, 6 + 4 * c);
-            r.slot[c] = __builtin_amdgcn_readlane(v, 7 + 4 * c);
-        }
-        return r;
-    };
-
-    // The first two children of an op.  A partials child loads its MFMA A
-    // operands: rows (4t + q) of P at column pl, and at column 16 + (pl & 3)
-    // (states 16..19; lanes pl >= 4 repeat them, which only fills output
-    // rows 4..15 of acc1, on lanes q > 0, cleared before use).  A tip child
-    // loads the P row of its code: entries 4q..4q+3 in R[0..3] and 16..19
-    // in R[6..9].  These loads depend on the program only, so an op's are
-    // issued while the op before it finishes (after its products, before
-    // its barrier); the op's HBM stores of the previous result always
-    // follow them, so no wait on them reaches back past those stores.
-    float R[2][10];
-    int kind[2];
-    unsigned code[2];
-    // An op with one child loads that child twice: every op issues the same
-    // twenty loads, so the wait counts the compiler derives do not depend
-    // on the path (a shorter path would lower them for all).
-    auto issueLoads = [&](const AaRec &op) {
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int cc = c < op.nKids ? c : 0;
-            const KidRec kd{op.kind[cc], op.idx[cc], op.pnode[cc], op.slot[cc]};
-            const bool tip = kd.kind == 0;
-            kind[c] = kd.kind;
-            const unsigned cd = tipCode(tip ? kd.idx : 0);
-            code[c] = cd;
-            const char *Pb = (const char *)PT + (size_t)(unsigned)(kd.pnode * K + k) * (AA_S * AA_S * 4);
-            if (tip) {
-                // two 16-byte loads per lane: a tip row touches one or two
-                // lines per pattern, and ten dword gathers would touch them
-                // five times over
-                const unsigned row = (cd < (unsigned)AA_S ? cd : 0u) * (AA_S * 4u);
-                const f4v v0 = *(const f4v *)(Pb + row + 16u * q);
-                const f4v v1 = *(const f4v *)(Pb + row + 64u);
-                for (int r = 0; r < 4; r++) {
-                    R[c][r] = v0[r];
-                    R[c][6 + r] = v1[r];
-                }
-            } else {
-                const unsigned o0 = (unsigned)(q * AA_S + pl) * 4u;
-                const unsigned o1 = (unsigned)(q * AA_S + 16 + (pl & 3)) * 4u;
-#pragma unroll
-                for (int t = 0; t < 5; t++) {
-                    R[c][t] = *(const float *)(Pb + 320 * t + o0);
-                    R[c][5 + t] = *(const float *)(Pb + 320 * t + o1);
-                }
-            }
-        }
-    };
-
-    double contrib = 0.0;
-    int bad = 0;
-    int par = 0;
-    bool sawRoot = false;
-    // the ops of all groups are contiguous, in program order (root last)
-    // Every op flushes a pending result (a fixed number of stores on every
-    // path, for the same reason).  The first op has none: it flushes the
-    // staging region (unwritten) to its own destination, which its real
-    // result overwrites one op later, in order, before anything reads it.
-    // Programs here have two or more ops, the root last.
-    const int nOps = a.nOps;
-    int recNext = recLoad(1);
-    AaRec op = recTake(recLoad(0));
-    pend = true;
-    pDst = op.dst;
-    pSrc = a.nLds;
-    issueLoads(op);
-    for (int i = 0; i < nOps; ++i) {
-        {
-            // the previous op's HBM stores, behind this op's loads
-            flush();
-            // products
-            f4v pr0 = zero, pr1 = zero;
-            int e = 0;
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                if (c >= op.nKids) break;
-                f4v v0, v1;
-                if (kind[c] == 0) {
-                    // a one-state code: its P row; all states: 1 (a product
-                    // with 1.0 leaves the other factor's bits unchanged, as
-                    // skipping it would); no branch on the lane's code
-                    const unsigned cd = code[c];
-                    const bool all = cd == TIP_ALL;
-                    for (int r = 0; r < 4; r++) {
-                        v0[r] = all ? 1.f : R[c][r];
-                        v1[r] = all ? 1.f : R[c][6 + r];
-                    }
-                    // partial ambiguity (rare): the sum of its states' P rows
-                    const bool amb = cd >= (unsigned)AA_S && !all;
-                    if (__builtin_amdgcn_ballot_w64(amb)) {
-                        if (amb) {
-                            const float *Pk = PT + ((size_t)op.pnode[c] * K + k) * AA_S * AA_S;
-                            const uint64_t m = a.ambMask[cd - AA_S];
-                            v0 = zero;
-                            v1 = zero;
-                            for (int j = 0; j < AA_S; j++)
-                                if ((m >> j) & 1ull) {
-                                    v0 += *reinterpret_cast<const f4v *>(Pk + j * AA_S + 4 * q);
-                                    v1 += *reinterpret_cast<const f4v *>(Pk + j * AA_S + 16);
-                                }
-                        }
-                        // settle the rare path's loads here (see the HBM branch below)
-                        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-                    }
-                } else {
-                    // (each branch reads through its own pointer: a pointer
-                    // chosen between LDS and HBM would become a flat access)
-                    const KidRec kd{op.kind[c], op.idx[c], op.pnode[c], op.slot[c]};
-                    f4v acc0 = zero, acc1 = zero;
-                    // (the products sit in each branch, so the HBM branch's
-                    // loads are consumed before the join and leave nothing
-                    // for the LDS branch to wait on)
-                    float b[5];
-                    if (kd.kind == 2) {
-                        const unsigned sr = (unsigned)(kd.pad * K + k);   // slot region
-                        const float *X = aaSlots + sr * 320u;
-                        e += slotEx[sr * AA_TILE + pl];
-#pragma unroll
-                        for (int t = 0; t < 5; t++) b[t] = X[t * 64 + lane];
-#pragma unroll
-                        for (int t = 0; t < 5; t++) {
-                            acc0 = mfma4(R[c][t], b[t], acc0);
-                            acc1 = mfma4(R[c][5 + t], b[t], acc1);
-                        }
-                    } else {
-                        const char *X =
-                            (const char *)(cl + (size_t)kd.idx * slotFloats + (size_t)tile * tileFloats + (size_t)k * 320);
-                        e += *(const int *)((const char *)(a.scl + (size_t)kd.idx * nPatPad + (size_t)tile * AA_TILE) + plB);
-#pragma unroll
-                        for (int t = 0; t < 5; t++) b[t] = *(const float *)(X + 256 * t + laneW);
-#pragma unroll
-                        for (int t = 0; t < 5; t++) {
-                            acc0 = mfma4(R[c][t], b[t], acc0);
-                            acc1 = mfma4(R[c][5 + t], b[t], acc1);
-                        }
-                        // settle this branch's loads here: left pending past the
-                        // join, they make the LDS branch wait on every
-                        // outstanding store as well (the wait counter is
-                        // merged across paths conservatively, so every rare
-                        // path that loads ends with such a wait)
-                        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-                    }
-                    v0 = acc0;
-                    v1 = acc1;
-                }
-                if (c == 0) {
-                    pr0 = v0;
-                    pr1 = v1;
-                } else {
-                    pr0 *= v0;
-                    pr1 *= v1;
-                }
-            }
-            // further children (a root with three or more) load and multiply in turn
-            for (int c = 2; c < op.nKids; ++c) {
-                const KidRec kd = kidAt(op.kidStart + c);
-                const float *Pk = PT + ((size_t)kd.pnode * K + k) * AA_S * AA_S;
-                f4v v0, v1;
-                bool skip = false;
-                if (kd.kind == 0) {
-                    const unsigned code = tipCode(kd.idx);
-                    skip = code == TIP_ALL;
-                    tipRow(Pk, code, v0, v1);
-                } else {
-                    f4v acc0 = zero, acc1 = zero;
-                    float b[5];
-                    if (kd.kind == 2) {
-                        const float *X = aaSlots + ((size_t)kd.pad * K + k) * 320;
-                        e += slotEx[((size_t)kd.pad * K + k) * AA_TILE + pl];
-#pragma unroll
-                        for (int t = 0; t < 5; t++) b[t] = X[t * 64 + lane];
-                    } else {
-                        const float *X = cl + (size_t)kd.idx * slotFloats + (size_t)tile * tileFloats + (size_t)k * 320;
-                        e += a.scl[(size_t)kd.idx * nPatPad + p];
-#pragma unroll
-                        for (int t = 0; t < 5; t++) b[t] = X[t * 64 + lane];
-                    }
-#pragma unroll
-                    for (int t = 0; t < 5; t++) {
-                        acc0 = mfma4(Pk[(4 * t + q) * AA_S + pl], b[t], acc0);
-                        acc1 = mfma4(Pk[(4 * t + q) * AA_S + 16 + (pl & 3)], b[t], acc1);
-                    }
-                    v0 = acc0;
-                    v1 = acc1;
-                }
-                if (!skip) {
-                    pr0 *= v0;
-                    pr1 *= v1;
-                }
-                __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): a rare path, settled here
-            }
-            if (q != 0) pr1 = zero;   // rows 4..15 of the states-16..19 products
-            // the next op's loads go out now (R is free), so their latency
-            // overlaps this op's barrier, rescale and result write
-            // (unconditional, past the end the last op again: every pass
-            // through the loop issues the same loads)
-            const AaRec cur = op;
-            op = recTake(recNext);
-            issueLoads(op);
-            recNext = recLoad(min(i + 2, nOps - 1));
-            // rescale: max over this wave's states, then over the categories
-            float m = 0.f;
-            for (int r = 0; r < 4; r++) m = fmaxf(m, fmaxf(pr0[r], pr1[r]));
-            m = fmaxf(m, __shfl_xor(m, 16));
-            m = fmaxf(m, __shfl_xor(m, 32));
-            if (q == 0) mx[par][k][pl] = m;
-            __syncthreads();
-            m = 0.f;
-            for (int kk = 0; kk < K; kk++) m = fmaxf(m, mx[par][kk][pl]);
-            par ^= 1;   // the next op posts into the other buffer: no second barrier
-            if (m < SCALE_THRESH && m > 0.f) {
-                int ex;
-                frexpf(m, &ex);
-                const int E = -ex;
-                for (int r = 0; r < 4; r++) {
-                    pr0[r] = ldexpf(pr0[r], E);
-                    pr1[r] = ldexpf(pr1[r], E);
-                }
-                e += E;
-            }
-            if (!(cur.flags & OP_ROOT)) {
-                // into the op's slot (the parent reads it there), or region
-                // nLds; the next op copies it to HBM
-                const int ld = (cur.flags >> 8) - 1;
-                const int dl = ld >= 0 ? ld : a.nLds;
-                float *L = aaSlots + ((size_t)dl * K + k) * 320;
-                for (int r = 0; r < 4; r++) L[(q * 4 + r) * AA_TILE + pl] = pr0[r];
-                if (q == 0) {
-                    for (int r = 0; r < 4; r++) L[(4 * 4 + r) * AA_TILE + pl] = pr1[r];
-                    slotEx[((size_t)dl * K + k) * AA_TILE + pl] = e;
-                }
-                pend = true;
-                pDst = cur.dst;
-                pSrc = dl;
-                continue;
-            }
-            // root: this category's sum_s pi_s cl_s across the four lanes of
-            // the pattern, then wave 0 adds the categories in order
-            const double *pi = a.rootPi;
-            uint64_t msk = ~0ull;
-            if (a.rootLeafRow >= 0) {
-                const unsigned code = tipCode(a.rootLeafRow);
-                msk = code < (unsigned)AA_S ? (1ull << code) : code == TIP_ALL ? ~0ull : a.ambMask[code - AA_S];
-            }
-            double Lk = 0.0;
-            for (int r = 0; r < 4; r++) {
-                const int s0i = 4 * q + r;
-                if ((msk >> s0i) & 1ull) Lk += pi[s0i] * (double)pr0[r];
-                if (q == 0 && ((msk >> (16 + r)) & 1ull)) Lk += pi[16 + r] * (double)pr1[r];
-            }
-            Lk += __shfl_xor(Lk, 16);
-            Lk += __shfl_xor(Lk, 32);
-            if (q == 0) rootL[k][pl] = Lk;
-            __syncthreads();
-            if (k == 0 && q == 0) {
-                double L = 0.0;
-                for (int kk = 0; kk < K; kk++) L += rootL[kk][pl];
-                rootL[0][pl] = L;   // the site term is taken after the loop, where its
-                rootE[pl] = e;      // constants do not occupy registers across it
-            }
-            sawRoot = true;
-            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the root's loads, settled here
-        }
-    }
-    if (pend) flush();
-    if (sawRoot && k == 0 && q == 0) siteLogLike<true>(a, rootL[0][pl], rootE[pl], p, K, a.rootPi, contrib, bad);
-    if (k == 0) finishSiteSumWave(a, contrib, bad, tile, nTiles);
-}
-
-// at most 102 VGPRs: five waves per SIMD, so prot128's 4,976 category
-// waves are resident in one round on 1,024 SIMDs (four per SIMD took two)
-template <bool TIPLDS>
-__global__ __launch_bounds__(64 * WAVE_MAX_K) __attribute__((amdgpu_waves_per_eu(5))) void k_pruneAaCat(PruneArgs a)
-{
-    pruneAaCatBody<TIPLDS>(a, blockIdx.x, gridDim.x);
-}
-
-// TIPLDS: every item of the launch stages its tip codes (items that could
-// are read from global memory by the other instance, which ignores tipLds)
-template <bool TIPLDS>
-__global__ __launch_bounds__(64 * WAVE_MAX_K) __attribute__((amdgpu_waves_per_eu(5))) void k_pruneAaCatBatch(
-    const PruneArgs *args, const int *blockItem)
-{
-    const int item = blockItem[2 * blockIdx.x];
-    const int local = blockItem[2 * blockIdx.x + 1];
-    const PruneArgs a = args[item];
-    pruneAaCatBody<TIPLDS>(a, local, a.nPatPad / AA_TILE);
-}
-
-// Category waves pay one barrier per op; short programs (dirty paths)
-// run faster on the tile kernel, long ones (full evaluations) on these.
-static int g_aaCat = 1;
-static int g_aaCatMinOps = AA_CAT_MIN_OPS;
-
-void setAaTuning(int catWaves, int minOps)
-{
-    g_aaCat = catWaves ? 1 : 0;
-    g_aaCatMinOps = minOps < 0 ? 0 : minOps;
-}
-
-bool pruneAaCategoryWaves(int nOps) { return g_aaCat != 0 && nOps >= std::max(2, g_aaCatMinOps); }
-
-// LDS slot file of the category kernel: per slot, K x (320 values + 16
-// exponents), and one more such region for a result without a slot.  Four
-// slots and that region for K = 4 take 26 KB, and the tip codes of up to
-// 128 taxa 2 KB more, so five workgroups (the five waves per SIMD the
-// kernel is built for) fit a CU's 160 KB.
-static int g_aaLdsSlots = 5;
-constexpr size_t AA_LDS_BUDGET = 28 * 1024;   // slots and the staging region
-void setAaLdsSlots(int n) { g_aaLdsSlots = n < 0 ? 0 : n; }
-int pruneAaLdsSlots(int K)
-{
-    const size_t per = (size_t)K * (320 + 16) * 4;
-    const size_t fit = AA_LDS_BUDGET / per;
-    return (int)std::min<size_t>((size_t)g_aaLdsSlots, fit > 0 ? fit - 1 : 0);
-}
-// the tile's tip codes go to LDS up to this many taxa (4 KB)
-constexpr int AA_TIP_LDS_MAX_TAXA = 256;
-bool pruneAaTipLds(int nTax) { return nTax <= AA_TIP_LDS_MAX_TAXA; }
-size_t pruneAaLdsBytes(int K, int nLds, int tipTaxa)
-{
-    return (size_t)(nLds + 1) * K * (320 + 16) * 4 + (size_t)tipTaxa * AA_TILE;
-}
-static bool aaLdsArgsOk(const PruneArgs &a)
-{
-    return a.nLds >= 0 && a.nLds <= pruneAaLdsSlots(a.K) && (!a.tipLds || pruneAaTipLds(a.nTax)) &&
-           a.aaRec != nullptr && a.nOps >= 2;
-}
-
-template <int KC>
-__global__ __launch_bounds__(PRUNE_THREADS) void k_pruneAaBatch(const PruneArgs *args, const int *blockItem)
-{
-    const int item = blockItem[2 * blockIdx.x];
-    const int local = blockItem[2 * blockIdx.x + 1];
-    const PruneArgs a = args[item];
-    pruneAaBody<KC>(a, local, a.nPatPad / (AA_TILE * PRUNE_THREADS / 64));
-}
-
-bool pruneUsesMfma(int dim, int K, int precision) { return dim == AA_S && precision == FP32 && K <= 8; }
-
-int pruneBlockPatternsFor(int dim, int K, int precision, int nOps)
-{
-    if (pruneUsesMfma(dim, K, precision))
-        return pruneAaCategoryWaves(nOps) ? AA_TILE : AA_TILE * PRUNE_THREADS / 64;
-    return pruneBlockPatterns(K);
-}
-
-static int aaKC(int K) { return K <= 1 ? 1 : K <= 2 ? 2 : K <= 4 ? 4 : 8; }
-
-hipError_t launchPruneAa(const PruneArgs &a, int nBlocks, hipStream_t s)
-{
-    if (pruneAaCategoryWaves(a.nOps)) {
-        if (a.K < 1 || a.K > WAVE_MAX_K || nBlocks * AA_TILE > a.nPatPad || !aaLdsArgsOk(a))
-            return hipErrorInvalidValue;
-        const size_t lds = pruneAaLdsBytes(a.K, a.nLds, a.tipLds ? a.nTax : 0);
-        if (a.tipLds)
-            hipLaunchKernelGGL(k_pruneAaCat<true>, dim3(nBlocks), dim3(64 * a.K), lds, s, a);
-        else
-            hipLaunchKernelGGL(k_pruneAaCat<false>, dim3(nBlocks), dim3(64 * a.K), lds, s, a);
-        return hipGetLastError();
-    }
-    if (nBlocks * AA_TILE * (PRUNE_THREADS / 64) > a.nPatPad) return hipErrorInvalidValue;
-    switch (aaKC(a.K)) {
-    case 1: hipLaunchKernelGGL(k_pruneAa<1>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, a); break;
-    case 2: hipLaunchKernelGGL(k_pruneAa<2>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, a); break;
-    case 4: hipLaunchKernelGGL(k_pruneAa<4>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, a); break;
-    default: hipLaunchKernelGGL(k_pruneAa<8>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, a); break;
-    }
-    return hipGetLastError();
-}
-
-bool pruneAaCatItemOk(const PruneArgs &a) { return aaLdsArgsOk(a); }
-
-hipError_t launchPruneAaBatch(const PruneArgs *d, const int *bi, int nBlocks, int K, bool catWaves, size_t ldsBytes,
-                              bool tipLds, hipStream_t s)
-{
-    if (catWaves) {
-        // every item of the launch has exactly K categories (the batch groups
-        // by K); ldsBytes: the largest slot file and tip codes of its items;
-        // tipLds: every item stages its tip codes
-        if (K < 1 || K > WAVE_MAX_K ||
-            ldsBytes > pruneAaLdsBytes(K, pruneAaLdsSlots(K), AA_TIP_LDS_MAX_TAXA))
-            return hipErrorInvalidValue;
-        if (tipLds)
-            hipLaunchKernelGGL(k_pruneAaCatBatch<true>, dim3(nBlocks), dim3(64 * K), ldsBytes, s, d, bi);
-        else
-            hipLaunchKernelGGL(k_pruneAaCatBatch<false>, dim3(nBlocks), dim3(64 * K), ldsBytes, s, d, bi);
-        return hipGetLastError();
-    }
-    switch (aaKC(K)) {
-    case 1: hipLaunchKernelGGL(k_pruneAaBatch<1>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, d, bi); break;
-    case 2: hipLaunchKernelGGL(k_pruneAaBatch<2>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, d, bi); break;
-    case 4: hipLaunchKernelGGL(k_pruneAaBatch<4>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, d, bi); break;
-    default: hipLaunchKernelGGL(k_pruneAaBatch<8>, dim3(nBlocks), dim3(PRUNE_THREADS), 0, s, d, bi); break;
-    }
-    return hipGetLastError();
-}
-
 // ------------------------------------------------ wave-per-category DNA
 // One wavefront per (64-pattern tile, gamma category); a workgroup holds
 // the K category waves of one tile and they share nothing but the staged
@@ -1989,10 +1241,6 @@ template <> struct Vec4T<float> { typedef float4 type; };
 template <> struct Vec4T<double> { typedef double4 type; };
 
 constexpr int WAVE_LDS_BUDGET = 48 * 1024;   // dynamic LDS per workgroup
-// s_waitcnt vmcnt(0) with the other counters left alone (gfx9 encoding:
-// vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
-constexpr int VMCNT0 = 0x0F70;
-
 // leafVec for 4 states with P^T in registers.  A single-state code (the
 // common case) picks its row with a 2-bit select tree; gaps, '?' and
 // partial ambiguities are fixed up on a divergent path that is skipped
@@ -2022,44 +1270,6 @@ __device__ __forceinline__ void leafVec4(const T *Pl, unsigned code, const uint6
                 v[s] = x;
             }
         }
-    }
-}
-
-// The last workgroup of the item sums the per-workgroup partials (wave 0
-// of each workgroup reports) in a fixed order with Neumaier compensation.
-__device__ __forceinline__ void finishSiteSumWave(const PruneArgs &a, double contrib, int bad, int blk, int nBlk)
-{
-    const int lane = threadIdx.x & 63;
-    for (int off = 32; off >= 1; off >>= 1) {
-        contrib += __shfl_xor(contrib, off);
-        bad |= __shfl_xor(bad, off);
-    }
-    unsigned prev = 0;
-    if (lane == 0) prev = postBlockSum(a, contrib, bad, blk);
-    prev = __shfl(prev, 0);
-    if (prev != (unsigned)(nBlk - 1)) return;
-    __threadfence();
-    double s = 0.0, comp = 0.0;
-    int b = 0;
-    for (int i = lane; i < nBlk; i += 64) {
-        const double x = __hip_atomic_load(a.blockSums + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        b |= __hip_atomic_load(a.blockBad + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const double t = s + x;  // Neumaier
-        if (fabs(s) >= fabs(x))
-            comp += (s - t) + x;
-        else
-            comp += (x - t) + s;
-        s = t;
-    }
-    double v = s + comp;
-    for (int off = 32; off >= 1; off >>= 1) {
-        v += __shfl_xor(v, off);
-        b |= __shfl_xor(b, off);
-    }
-    if (lane == 0) {
-        a.result[0] = b ? -1.0e99 : v;
-        a.result[1] = (double)b;
-        *a.counter = 0u;
     }
 }
 

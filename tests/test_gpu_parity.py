@@ -565,3 +565,79 @@ def test_batch_error_keeps_staged_p_matrices():
         got = pf.p4_getBigPDeck(a.nodes[nn].cNode, p, mp.nGammaCat, mp.dim)
         want = pf.p4_getBigPDeck(ctrl.nodes[nn].cNode, p, mp.nGammaCat, mp.dim)
         assert numpy.array_equal(got, want), p
+
+
+def _newick(shape, n):
+    """n leaves t0.. as a caterpillar, a balanced tree, or a tree whose root
+    and one other node have five children."""
+    L = ["t%d:0.%02d" % (i, 5 + i % 40) for i in range(n)]
+    if shape == "caterpillar":
+        s = L[0]
+        for x in L[1:-2]:
+            s = "(%s,%s):0.03" % (s, x)
+        return "(%s,%s,%s);" % (s, L[-2], L[-1])
+    if shape == "polytomy":
+        return "(%s,(%s):0.07,%s);" % (",".join(L[:2]), ",".join(L[2:7]), ",".join(L[7:]))
+    while len(L) > 3:
+        L = ["(%s,%s):0.04" % (L[i], L[i + 1]) if i + 1 < len(L) else L[i] for i in range(0, len(L), 2)]
+    return "(%s);" % ",".join(L)
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", FP64_TOL), ("fp32", FP32_TOL)])
+@pytest.mark.parametrize("shape,nTax,nPat,nCat", [
+    ("caterpillar", 3, 1, 1), ("caterpillar", 40, 16, 8), ("balanced", 128, 33, 4), ("balanced", 300, 17, 2),
+    ("polytomy", 10, 300, 4), ("polytomy", 14, 5, 5)])
+def test_protein_kernel_edges_match_oracle(prec, tol, shape, nTax, nPat, nCat):
+    """The 20-state kernel at its edges: one op only, one tile and a pattern
+    more, one to eight categories, more taxa than its LDS tip codes hold, a
+    tree that needs more LDS slots than it has (results read back from HBM),
+    and nodes of five children; then with a few branches changed and only
+    their paths recomputed, one after the other and, batched, together."""
+    from p4gpu import Data, Part, func
+    rng = numpy.random.default_rng(nTax + nPat)
+    t = func.readNewick(_newick(shape, nTax))
+    names = ["t%d" % i for i in range(nTax)]
+    t.taxNames = names
+    codes = numpy.where(rng.random((nTax, nPat)) < 0.7, rng.integers(0, 20, nPat)[None, :],
+                        rng.integers(0, 20, (nTax, nPat)))
+    hit = rng.random(codes.shape) < 0.1
+    codes[hit] = rng.choice(numpy.array([-1, -2, -64, -63, -62]), size=int(hit.sum()))
+    t.data = Data(parts=[Part.fromPatterns(codes, rng.integers(1, 9, nPat), "protein")], taxNames=names)
+    t.newComp(free=1, spec="specified", val=list(rng.dirichlet(numpy.full(20, 5.0))))
+    t.newRMatrix(free=1, spec="specified", val=list(rng.lognormal(0, 1, 190)))
+    t.setNGammaCat(nGammaCat=nCat)
+    if nCat > 1:
+        t.newGdasrv(free=1, val=0.7)
+    t.setPInvar(free=1, val=0.1)
+    t.setPrecision(prec)
+    trees = [t, t.dupe()]
+    for x in trees:
+        v = x.calcLogLike(verbose=0)
+        assert rel(v, oracle.part_loglike(oracle.flat_from_tree(x, 0))) < tol
+    batch = pf.Batch([x.cTree for x in trees])
+    kids = [n.nodeNum for n in t.iterNodesNoRoot()]
+    for step in range(4):
+        for x in trees:
+            n = x.nodes[kids[int(rng.integers(len(kids)))]]
+            n.br.len = float(rng.uniform(0.01, 0.5))
+            pf.p4_setBrLen(n.cNode, n.br.len)
+            pf.p4_calculateBigPDecks(n.cNode)
+            pf.markPath(x.cTree, n.parent.nodeNum, -1)
+        got = batch.logLikes() if step % 2 else [pf.p4_partLogLike(x.cTree, x.data.parts[0].cPart, 0, 0) for x in trees]
+        for x, v in zip(trees, got):
+            assert rel(v, oracle.part_loglike(oracle.flat_from_tree(x, 0))) < tol, (step, v)
+
+
+def test_protein_operands_follow_a_copy_between_precisions():
+    """p4_copyBigPDecks between trees of different precision: the copied P
+    matrices serve the destination's own kernel."""
+    a, _ = synth.make_workload("prot128", seed=4, nSites=60)
+    b = a.dupe()
+    a.setPrecision("fp64")
+    b.setPrecision("fp32")
+    for n in b.iterNodesNoRoot():
+        n.br.len *= 2.0
+    va = a.calcLogLike(verbose=0)
+    b.calcLogLike(verbose=0)
+    pf.p4_copyBigPDecks(a.cTree, b.cTree, 1)
+    assert rel(pf.p4_treeLogLike(b.cTree, 0), va) < FP32_TOL
