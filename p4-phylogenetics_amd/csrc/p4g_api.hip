@@ -187,6 +187,7 @@ static void freeTreePart(TreePart &t)
     devFree(t.P1T);
     devFree(t.P2T);
     devFree(t.dQ);
+    devFree(t.dD);
     devFree(t.dRate);
     devFree(t.dPartial);
     devFree(t.dOut);
@@ -1778,6 +1779,7 @@ static bool derivPart(Tree *t, int pNum, std::vector<double> &out)
     const size_t SS = (size_t)S * S;
     if (!devAlloc(&tp.cl2, (size_t)N * K * tp.nPatPad * S, "hipMalloc cl2") ||
         !devAlloc(&tp.P1T, (size_t)N * K * SS, "hipMalloc P'") || !devAlloc(&tp.P2T, (size_t)N * K * SS, "hipMalloc P''") ||
+        (tp.mfma && !devAlloc(&tp.dD, (size_t)N * K * 3 * AA_MAT, "hipMalloc P' operands")) ||
         !devAlloc(&tp.dQ, (size_t)std::max(tp.nEig, 1) * SS, "hipMalloc Q") ||
         !devAlloc(&tp.dRate, (size_t)N * K, "hipMalloc rate factors") ||
         !devAlloc(&tp.dItems, (size_t)2 * N, "hipMalloc derivative items") ||
@@ -1830,9 +1832,65 @@ static bool derivPart(Tree *t, int pNum, std::vector<double> &out)
         op.nSib = (int)sibs.size() - op.sibStart;
         ops.push_back(op);
     }
+    const int layout = tp.wave ? CL_WAVE : tp.mfma ? CL_TILED : CL_GROUPED;
+    // the unit kernels: every internal node in preorder, its children's
+    // branches together (two children) or one by one; ops in that order
+    std::vector<DerivUnit> units;
+    if (derivUsesUnits(S, K, layout)) {
+        std::vector<int> opOf(N, -1), itemOf(N, 0);
+        for (int i = 0; i < nI; i++) itemOf[items[i]] = i;
+        for (size_t i = 0; i < ops.size(); i++) opOf[ops[i].node] = (int)i;
+        std::vector<DerivOp> ordered;
+        std::vector<int> nodes;   // the parents, each before its children's children
+        for (int j = N - 1; j >= 0; j--) {
+            const int n = t->postOrder[j];
+            if (n != NO_ORDER && t->nodes[n]->leftChild >= 0) nodes.push_back(n);
+        }
+        int prevNode[2] = {-1, -1};
+        for (int m : nodes) {
+            std::vector<int> kids;
+            for (int c = t->nodes[m]->leftChild; c >= 0; c = t->nodes[c]->sibling) kids.push_back(c);
+            const size_t step = kids.size() == 2 ? 2 : 1;
+            for (size_t c = 0; c < kids.size(); c += step) {
+                DerivUnit u{};
+                u.nKids = (int)step;
+                u.parent = m;
+                u.src = m == t->root ? DU_ROOT : m == prevNode[0] ? DU_PREV0 : m == prevNode[1] ? DU_PREV1 : DU_HBM;
+                u.out = (int)ordered.size();
+                prevNode[1] = -1;
+                for (size_t i = 0; i < step; i++) {
+                    const DerivOp &o = ops[opOf[kids[c + i]]];
+                    u.node[i] = o.node;
+                    u.tip[i] = (o.flags & DOP_LEAF) ? 1 : 0;
+                    u.idx[i] = o.idx;
+                    u.item[i] = itemOf[o.node];
+                    u.eig[i] = items[N + itemOf[o.node]];
+                    if (step == 1) {
+                        u.sibStart = o.sibStart;
+                        u.nSib = o.nSib;
+                    }
+                    prevNode[i] = o.node;
+                    ordered.push_back(o);
+                }
+                if (step == 1) {
+                    u.node[1] = u.node[0];
+                    u.tip[1] = u.tip[0];
+                    u.idx[1] = u.idx[0];
+                }
+                units.push_back(u);
+            }
+        }
+        if (ordered.size() != ops.size()) {
+            setError("branch derivatives: the postorder does not reach every node");
+            return false;
+        }
+        ops.swap(ordered);
+    }
     const int nOps = (int)ops.size();
-    const int nBlocks = tp.nPatPad / 64;
-    const size_t progBytes = ops.size() * sizeof(DerivOp) + std::max<size_t>(sibs.size(), 1) * sizeof(DerivSib);
+    const int nBlocks = tp.nPatPad / derivBlockPatterns(S, K, layout);
+    // units first: each is one aligned 64-byte record
+    const size_t progBytes = units.size() * sizeof(DerivUnit) + ops.size() * sizeof(DerivOp) +
+                             std::max<size_t>(sibs.size(), 1) * sizeof(DerivSib);
     if (progBytes > tp.dProgCap) {
         if (tp.dProg) (void)hipFree(tp.dProg);
         tp.dProg = nullptr;
@@ -1845,19 +1903,24 @@ static bool derivPart(Tree *t, int pNum, std::vector<double> &out)
         if (!devAlloc(&tp.dPartial, partN, "hipMalloc derivative sums")) return false;
         tp.dPartialCap = partN;
     }
-    DerivOp *dOps = reinterpret_cast<DerivOp *>(tp.dProg);
+    DerivUnit *dUnits = reinterpret_cast<DerivUnit *>(tp.dProg);
+    DerivOp *dOps = reinterpret_cast<DerivOp *>(dUnits + units.size());
     DerivSib *dSibs = reinterpret_cast<DerivSib *>(dOps + ops.size());
     if (!hipOk(hipMemcpyAsync(tp.dQ, Q.data(), Q.size() * 8, hipMemcpyHostToDevice, s), "stage Q") ||
         !hipOk(hipMemcpyAsync(tp.dRate, rate.data(), rate.size() * 8, hipMemcpyHostToDevice, s), "stage rates") ||
         !hipOk(hipMemcpyAsync(tp.dItems, items.data(), items.size() * 4, hipMemcpyHostToDevice, s), "stage items") ||
         !hipOk(hipMemcpyAsync(dOps, ops.data(), ops.size() * sizeof(DerivOp), hipMemcpyHostToDevice, s), "stage program") ||
+        (!units.empty() &&
+         !hipOk(hipMemcpyAsync(dUnits, units.data(), units.size() * sizeof(DerivUnit), hipMemcpyHostToDevice, s),
+                "stage program")) ||
         (!sibs.empty() &&
          !hipOk(hipMemcpyAsync(dSibs, sibs.data(), sibs.size() * sizeof(DerivSib), hipMemcpyHostToDevice, s),
                 "stage siblings"))) {
         (void)hipStreamSynchronize(s);
         return false;
     }
-    DerivPArgs pa{S, K, nI, tp.dItems, tp.dItems + N, tp.dRate, tp.dQ, tp.PT64, tp.P1T, tp.P2T};
+    DerivPArgs pa{S, K, nI, tp.dItems, tp.dItems + N, tp.dRate, tp.dQ, tp.PT64, tp.P1T, tp.P2T,
+                  tp.dD};
     if (!hipOk(launchPderiv(pa, s), "launch P derivative kernel")) {
         (void)hipStreamSynchronize(s);
         return false;
@@ -1868,9 +1931,17 @@ static bool derivPart(Tree *t, int pNum, std::vector<double> &out)
     a.nPat = tp.nPat;
     a.nPatPad = tp.nPatPad;
     a.nOps = nOps;
-    a.layout = tp.wave ? CL_WAVE : tp.mfma ? CL_TILED : CL_GROUPED;
+    a.layout = layout;
     a.ops = dOps;
     a.sibs = dSibs;
+    a.nUnits = (int)units.size();
+    a.units = dUnits;
+    a.PA = reinterpret_cast<const double *>(tp.PA);
+    a.D = tp.dD;
+    a.Q = tp.dQ;
+    a.rateFac = tp.dRate;
+    a.nTax = dp->nTax;
+    a.nAmb = dp->dev.nAmb;
     a.tips = dp->dev.tips;
     a.ambMask = dp->dev.ambMask;
     a.cl = reinterpret_cast<const double *>(tp.cl);
@@ -3100,7 +3171,10 @@ int p4g_getCondLikes2(const p4g_node *n, int pNum, double *out)
         return 1;
     for (int k = 0; k < K; k++)
         for (int s = 0; s < S; s++)
-            for (int p = 0; p < nP; p++) out[((size_t)k * S + s) * nP + p] = v[((size_t)k * tp.nPatPad + p) * S + s];
+            for (int p = 0; p < nP; p++)
+                out[((size_t)k * S + s) * nP + p] =
+                    tp.mfma ? v[((size_t)(p / AA_TILE) * K + k) * AA_PART + aaIndex(s, p % AA_TILE, false)]
+                            : v[((size_t)k * tp.nPatPad + p) * S + s];
     return 0;
 }
 

@@ -348,7 +348,7 @@ struct TreePart {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double lastKernelUs = -1.0;
     // branch-length derivatives (allocated by their first use)
-    double *cl2 = nullptr, *P1T = nullptr, *P2T = nullptr, *dQ = nullptr, *dRate = nullptr;
+    double *cl2 = nullptr, *P1T = nullptr, *P2T = nullptr, *dQ = nullptr, *dRate = nullptr, *dD = nullptr;
     double *dPartial = nullptr, *dOut = nullptr;
     int *dItems = nullptr;
     void *dProg = nullptr;
@@ -467,6 +467,23 @@ struct DerivOp {
 struct DerivSib {
     int kind, idx, pnode, pad;   // kind 0 tip (idx: tip row), 1 internal (idx: partials slot)
 };
+// The 4-state (wave layout) and 20-state (tiles) kernels walk units in
+// preorder instead: a node with two children, both of whose branches are
+// done together, or (any other number of children) one child at a time.
+enum { DU_ROOT = 0, DU_HBM = 1, DU_PREV0 = 2, DU_PREV1 = 3 };
+struct DerivUnit {
+    int nKids;       // 2: children 0 and 1; 1: child 0 (repeated as 1), its siblings in the side array
+    int src;         // the parent's cl2: none (it is the root), HBM, or the previous unit's child 0 or 1
+    int parent;
+    int out;         // index of child 0's sums (child 1's follow)
+    int node[2];
+    int tip[2];      // 1 a leaf
+    int idx[2];      // tip row or partials slot
+    int sibStart, nSib;
+    int item[2];     // index of each child's rate factors
+    int eig[2];      // and its (comp, rMatrix) slot
+};
+static_assert(sizeof(DerivUnit) == 64, "DerivUnit is one 64-byte scalar load");
 constexpr int DERIV_MAX_K = 16;
 struct DerivPArgs {
     int dim, K, nItems;
@@ -476,12 +493,18 @@ struct DerivPArgs {
     const double *Q;             // [nEig][dim][dim] normalised rate matrices
     const double *PT64;          // P^T of the tree part
     double *P1T, *P2T;           // P'^T and P''^T, same layout
+    double *D;                   // 20-state operand tables of P^T, P' and P'' ([node][cat][3][400], aaPaIndex), or null
 };
 struct DerivArgs {
     int dim, K, nPat, nPatPad, nOps;
     int layout;                  // of the down-pass partials (CL_*)
     const DerivOp *ops;
     const DerivSib *sibs;
+    int nUnits;                  // the unit kernels (ops then gives the order of the sums only)
+    const DerivUnit *units;
+    const double *PA, *D;        // 20-state operand tables of P, and of P^T, P' and P''
+    const double *Q, *rateFac;   // of k_pderiv
+    int nTax, nAmb;
     const uint8_t *tips;
     const uint64_t *ambMask;
     const double *cl;            // FP64 down-pass partials
@@ -497,6 +520,8 @@ struct DerivArgs {
     double *out;                 // [nNodes][3]: lnL across the node's branch, d1, d2
 };
 hipError_t launchPderiv(const DerivPArgs &a, hipStream_t s);
+bool derivUsesUnits(int dim, int K, int layout);
+int derivBlockPatterns(int dim, int K, int layout);   // patterns per workgroup
 hipError_t launchEdgeDerivs(const DerivArgs &a, int nBlocks, hipStream_t s);
 
 // Kernel launchers (p4g_kernels.hip).

@@ -169,3 +169,49 @@ def test_derivatives_need_fp64_partials():
     tree.calcLogLike(verbose=0)
     with pytest.raises(P4Error, match="FP64"):
         tree.branchDerivatives()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dataType", ["dna", "protein"])
+@pytest.mark.parametrize("newick,nPat,nCat", [
+    ("(a:0.1,b:0.2,c:0.3);", 1, 1), ("((a:0.1,b:0.2):0.05,(c:0.3,d:0.1):0.2);", 65, 8),
+    ("((a:0.1,b:0.2,(c:0.1,d:0.3):0.04,e:0.2):0.05,((f:0.3,g:0.1):0.2,h:0.15):0.3,i:0.2,(j:0.1,k:0.1):0.02);", 33, 4),
+    ("(((((a:0.1,b:0.2):0.1,c:0.1):0.1,d:0.2):0.05,e:0.1):0.1,f:0.3,g:0.1);", 300, 9)])
+def test_derivatives_on_odd_trees(dataType, newick, nPat, nCat):
+    """Two children at the root and nodes of four, chains, one tile and a
+    pattern more, one to nine categories (nine: the general kernel), gaps
+    and ambiguities: the likelihood across every branch is the tree's, and
+    d1 and d2 are finite differences of it (tolerances of the tests above)."""
+    from p4gpu import Data, Part, func
+    rng = numpy.random.default_rng(nPat)
+    t = func.readNewick(newick)
+    names = [n.name for n in t.iterLeavesNoRoot()]
+    t.taxNames = names
+    S = 4 if dataType == "dna" else 20
+    codes = numpy.where(rng.random((len(names), nPat)) < 0.7, rng.integers(0, S, nPat)[None, :],
+                        rng.integers(0, S, (len(names), nPat)))
+    hit = rng.random(codes.shape) < 0.15
+    codes[hit] = rng.choice(numpy.array([-1, -2, -64, -63, -62]), size=int(hit.sum()))
+    t.data = Data(parts=[Part.fromPatterns(codes, rng.integers(1, 9, nPat), dataType)], taxNames=names)
+    for _ in range(2):
+        t.newComp(free=1, spec="specified", val=list(rng.dirichlet(numpy.full(S, 5.0))))
+    t.newRMatrix(free=1, spec="specified", val=list(rng.lognormal(0, 1, S * (S - 1) // 2)))
+    t.setNGammaCat(nGammaCat=nCat)
+    if nCat > 1:
+        t.newGdasrv(free=1, val=0.7)
+    t.setPInvar(free=1, val=0.1)
+    for i, n in enumerate(t.nodes):
+        n.parts[0].compNum = i % 2
+    v = t.calcLogLike(verbose=0)
+    lnl, d1, d2 = t.branchDerivatives()
+    for n in t.iterNodesNoRoot():
+        t0 = n.br.len
+        assert abs(lnl[n.nodeNum] - v) <= 1e-10 * abs(v), n.nodeNum
+
+        def at(x):
+            n.br.len = x
+            return t.calcLogLike(verbose=0)
+        f1, f2 = _fd(at, t0, 1e-4 * max(t0, 1e-2))
+        n.br.len = t0
+        assert abs(f1 - d1[n.nodeNum]) <= 1e-5 * max(1.0, abs(d1[n.nodeNum])), (n.nodeNum, f1, d1[n.nodeNum])
+        assert abs(f2 - d2[n.nodeNum]) <= 1e-2 * max(1.0, abs(d2[n.nodeNum])), (n.nodeNum, f2, d2[n.nodeNum])
