@@ -600,10 +600,10 @@ static void stageParams(Tree *t, int pNum)
     const int dim = t->model->parts[pNum]->dim;
     int nI = 0;
     for (int n = 0; n < t->nNodes; n++) nI += tp.pPending[n] ? 1 : 0;
-    // 20-state P straight from exp(Qt) is one latency-bound wavefront per
-    // matrix: worth it for many matrices (a Q change, a full evaluation),
-    // not for the few of a branch move, which reuse cached eigensystems
-    const bool direct = pmatDirect(dim) && (dim == 4 || nI >= PEXP_WAVE_MIN_ITEMS);
+    // (also for the few matrices of a branch move: the direct launch over 32
+    // partitions takes 18 us where the eigen route's P kernel takes 17 and,
+    // after a change of the model, 277 for the eigensystems)
+    const bool direct = pmatDirect(dim);
     tp.flushDirect = direct;
     if (!direct && tp.eigStale) {
         for (int i = 0; i < tp.nEig; i++)
@@ -1612,8 +1612,9 @@ static bool stagePart(Tree *t, int pNum, bool full, int *nOps, std::vector<Defer
     if (!tp.progOnDevice) need(tp.offProg, tp.offProg + sizeof(int) * tp.progWords);
     // 20-state P straight from exp(Qt) for many matrices: its (pi, R)
     // snapshots and the pack (the arena's first bytes) go up in the same
-    // copy (a few matrices read them across PCIe sooner than a copy runs)
-    const bool devEig = tp.flushDirect && mp->dim == 20 && tp.pendI * mp->nCat >= 64;
+    // copy.  A few matrices read them across PCIe sooner than a copy runs,
+    // unless a batched call's one upload launch carries them anyway.
+    const bool devEig = tp.flushDirect && mp->dim == 20 && tp.pendI > 0 && (uploads || tp.pendI * mp->nCat >= 64);
     if (devEig) need(0, tp.offPack + tp.packBytes);   // snapshots, eigen list and the pack
     if (hi > lo) {
         if (uploads)
@@ -3758,20 +3759,27 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
         std::copy(uploads.begin(), uploads.end(), b->hRanges);
         return hipOk(launchCopyRanges(b->dRanges, (int)uploads.size(), stream()), "launch upload kernel");
     };
+    // a later item failed to stage: the items before it get their uploads and
+    // then their P matrices (whose kernels read what the uploads bring; without
+    // them only those that read the pinned arena are launched)
+    auto failStaged = [&]() {
+        const std::string first = g_err;   // stays the reported error
+        if (!launchUploads())
+            defer.erase(std::remove_if(defer.begin(), defer.end(), [](const DeferredP &d) { return d.devIn != nullptr; }),
+                        defer.end());
+        launchDeferredEach(defer);
+        setError(first);
+    };
     for (size_t i = 0; i < b->trees.size(); i++) {
         Tree *t = b->trees[i];
         if (!treeReady(t)) {
-            launchDeferredEach(defer);
-            (void)launchUploads();
-            (void)hipStreamSynchronize(stream());
+            failStaged();
             return 1;
         }
         for (int p = 0; p < t->nParts; p++) {
             int nOps = 0;
             if (!stagePart(t, p, false, &nOps, &defer, &uploads)) {
-                launchDeferredEach(defer);
-                (void)launchUploads();
-                (void)hipStreamSynchronize(stream());
+                failStaged();
                 return 1;
             }
             items.push_back({t, p, nOps, (int)i});

@@ -531,7 +531,7 @@ hipError_t launchPmat(const PmatArgs &a, hipStream_t s);
 // prefix sums of each item's nItems * K * dim * dim entries).
 hipError_t launchPmatMulti(const PmatArgs *args, const int *first, int nItems, int total, hipStream_t s);
 // P = exp(Q t) per (branch, category) straight from the (pi, R) snapshots
-// eigIn (4-state parts only); pmatDirect(dim) says whether that route is on.
+// eigIn (4- and 20-state parts); pmatDirect(dim) says whether that route is on.
 hipError_t launchPexp(const PmatArgs &a, const double *eigIn, hipStream_t s);
 bool pmatDirect(int dim);
 // the 20-state kernel's operand table of n matrices from a.PT64
@@ -541,8 +541,6 @@ hipError_t launchAaOperands(const PmatArgs &a, int n, hipStream_t s);
 // sums of each item's nItems * K matrices, first[nItems] == total).
 hipError_t launchPexpMulti(int dim, const PmatArgs *args, const double *const *ins, const int *first, int nItems,
                            int total, hipStream_t s);
-// 20-state flushes with fewer pending P matrices use the eigen route.
-constexpr int PEXP_WAVE_MIN_ITEMS = 16;
 void setPmatRoute(int direct);
 hipError_t launchPrune(const PruneArgs &a, int precision, int nBlocks, hipStream_t s);
 hipError_t launchPruneBatch(const PruneArgs *dArgs, const int *dBlockItem, int nBlocks,

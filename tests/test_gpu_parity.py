@@ -395,6 +395,50 @@ def test_direct_p_extreme_branch_lengths():
                 assert (numpy.abs(got - want)[off] / want[off]).max() < 1e-12, (L, k)
 
 
+@pytest.mark.parametrize("direct,batched,nMoved", [(True, False, 1), (True, True, 1), (True, False, 8), (True, True, 8),
+                                                   (False, True, 1)])
+def test_protein_p_of_few_branches(direct, batched, nMoved):
+    """20-state P of one moved branch and of eight, from 1e-9 to 200
+    substitutions per site, after a full evaluation: alone (inputs read from
+    pinned memory) and in a batched call (inputs uploaded with the program),
+    against the exponential series in extended precision (short branches,
+    off-diagonal entries to 1e-13 of the largest) and scipy's expm; the eigen
+    route of a batched call to its own rounding (2e-14 at ordinary lengths,
+    condition times epsilon)."""
+    fx = load("prot128_150")
+    K, S = int(fx["nCat"]), int(fx["dim"])
+    lens = ([0.05, 1e-9, 200.0, 1e-5, 20.0, 1e-3, 0.7, 3.0])[:nMoved]
+    off = ~numpy.eye(S, dtype=bool)
+    try:
+        t = tree_from_fixture(fx, "fp64")
+        t.calcLogLike(verbose=0)
+        pf.setPmatRoute(direct)
+        nodes = [n for n in range(1, len(fx["parent"])) if n != int(fx["root"])][:nMoved]
+        for n, L in zip(nodes, lens):
+            pf.p4_setBrLen(t.nodes[n].cNode, L)
+            pf.p4_calculateBigPDecks(t.nodes[n].cNode)
+        if batched:
+            pf.Batch([t.cTree]).logLikes()
+        for n, L in zip(nodes, lens):
+            got = pf.p4_getBigPDeck(t.nodes[n].cNode, 0, K, S)
+            Q = _bigq_normalised(numpy.asarray(fx["comps"][int(fx["compNums"][n])], float),
+                                 numpy.asarray(fx["bigR"][int(fx["rMatrixNums"][n])], float))
+            for k in range(K):
+                tk = L * float(fx["rates"][int(fx["gdasrvNums"][n])][k]) * float(fx["relRate"]) / (1.0 - float(fx["pInvar"]))
+                tol = (1e-14 if tk < 5 else 1e-11) if direct else 1e-13
+                assert numpy.abs(got[k] - scipy_expm(Q * tk)).max() < tol, (L, k)
+                assert numpy.allclose(got[k].sum(1), 1.0, rtol=0, atol=1e-13)
+                if direct and tk < 1e-2:
+                    A = Q.astype(numpy.longdouble) * numpy.longdouble(tk)
+                    term, want = A, A
+                    for j in range(2, 16):
+                        term = term @ A / j
+                        want = want + term
+                    assert numpy.abs(got[k] - want)[off].max() < 1e-13 * want[off].max(), (L, k)
+    finally:
+        pf.setPmatRoute(True)
+
+
 @pytest.mark.parametrize("nCat", [4, 3])
 def test_protein_category_waves_match_tile_waves(nCat):
     """The 20-state MFMA kernel with one wavefront per (tile, category)
