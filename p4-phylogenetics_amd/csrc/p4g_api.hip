@@ -704,11 +704,14 @@ static bool launchParams(Tree *t, int pNum, std::vector<DeferredP> *defer = null
     return true;
 }
 
-static bool flushParams(Tree *t, int pNum)
+// queued: set when a kernel was launched (it reads the pinned arena, which
+// must not be written until it has run).
+static bool flushParams(Tree *t, int pNum, bool *queued = nullptr)
 {
     stageParams(t, pNum);
     TreePart &tp = t->tp[pNum];
     if (!tp.pendE && !tp.pendI) return true;
+    if (queued) *queued = true;
     return launchParams(t, pNum);
 }
 
@@ -2894,12 +2897,15 @@ int p4g_syncChanged(p4g_tree *a, p4g_tree *b)
         return 1;
     }
     hipStream_t s = stream();
-    // P matrices still pending in src are computed first
+    // P matrices still pending in src are computed first (and waited for:
+    // their kernels read a's pinned arena, which the next call may write)
+    bool queued = false;
     for (int p = 0; p < a->nParts; p++)
-        if (!flushParams(a, p)) {
+        if (!flushParams(a, p, &queued)) {
             (void)hipStreamSynchronize(s);
             return 1;
         }
+    if (queued && !hipOk(hipStreamSynchronize(s), "parameter kernels")) return 1;
     std::vector<CopyRange> r;
     for (int p = 0; p < a->nParts; p++) {
         TreePart &A = a->tp[p], &B = b->tp[p];
@@ -2971,8 +2977,19 @@ int p4g_copyModelPrams(p4g_tree *a, p4g_tree *b)
 {
     clearError();
     if (!a || !b || a->model->nParts != b->model->nParts) return 1;
-    if ((a->tp[0].alloc && !flushAll(a)) || (b->tp[0].alloc && !flushAll(b))) return 1;
+    // P matrices pending in either tree are computed first, and waited for:
+    // their kernels read the pinned arenas that the copy below writes.  With
+    // none pending (the reject step of a chain, whose evaluation computed
+    // them) nothing is waited for, so a queued state sync runs on meanwhile.
     hipStream_t s = stream();
+    bool queued = false;
+    for (Tree *t : {a, b})
+        for (int p = 0; p < t->nParts && t->tp[0].alloc; p++)
+            if (t->tp[p].alloc && !flushParams(t, p, &queued)) {
+                (void)hipStreamSynchronize(s);
+                return 1;
+            }
+    if (queued && !hipOk(hipStreamSynchronize(s), "parameter kernels")) return 1;
     for (int p = 0; p < a->model->nParts; p++) {
         ModelPart *A = a->model->parts[p], *B = b->model->parts[p];
         const int dim = A->dim;
@@ -2987,9 +3004,13 @@ int p4g_copyModelPrams(p4g_tree *a, p4g_tree *b)
         TreePart &TA = a->tp[p], &TB = b->tp[p];
         if (TA.alloc && TB.alloc && TA.nEig == TB.nEig) {
             const size_t ne = (size_t)TA.nEig;
-            if (!hipOk(hipMemcpyAsync(TB.eigV, TA.eigV, ne * dim * dim * 8, hipMemcpyDeviceToDevice, s), "copy eig") ||
-                !hipOk(hipMemcpyAsync(TB.eigVi, TA.eigVi, ne * dim * dim * 8, hipMemcpyDeviceToDevice, s), "copy eig") ||
-                !hipOk(hipMemcpyAsync(TB.eigLam, TA.eigLam, ne * dim * 8, hipMemcpyDeviceToDevice, s), "copy eig"))
+            // (stale eigensystems are not copied: the first flush that needs
+            // one recomputes every slot from the snapshots.  The three copies
+            // of each of 24 partitions took 250 us of a chain's reject step.)
+            if (!TA.eigStale &&
+                (!hipOk(hipMemcpyAsync(TB.eigV, TA.eigV, ne * dim * dim * 8, hipMemcpyDeviceToDevice, s), "copy eig") ||
+                 !hipOk(hipMemcpyAsync(TB.eigVi, TA.eigVi, ne * dim * dim * 8, hipMemcpyDeviceToDevice, s), "copy eig") ||
+                 !hipOk(hipMemcpyAsync(TB.eigLam, TA.eigLam, ne * dim * 8, hipMemcpyDeviceToDevice, s), "copy eig")))
                 return 1;
             // the (pi, R) snapshots go with the eigensystems: P of tree b
             // may be computed from them directly

@@ -439,6 +439,40 @@ def test_protein_p_of_few_branches(direct, batched, nMoved):
         pf.setPmatRoute(True)
 
 
+@pytest.mark.parametrize("stale", [True, False])
+def test_copied_model_serves_the_eigen_route(stale):
+    """p4_copyModelPrams of a tree whose eigensystems are stale (P came
+    straight from the snapshots) or computed (eigen route): a branch moved on
+    the receiving tree gets, on the eigen route, the giving tree's P (to the
+    eigen route's rounding, as in the tests above), also right after a queued
+    state sync."""
+    t = synth.make_workload("multi48", seed=5, nSites=700, precision="fp64")[0]
+    try:
+        u = t.dupe()
+        u.calcLogLike(verbose=0)
+        n = list(t.iterNodesNoRoot())[3]
+        old = [pf.p4_getBigPDeck(u.nodes[n.nodeNum].cNode, p, mp.nGammaCat, mp.dim) for p, mp in enumerate(u.model.parts)]
+        pf.setPmatRoute(stale)
+        for mp in t.model.parts:
+            mp.rMatrices[0].val = mp.rMatrices[0].val * numpy.linspace(0.5, 2.0, len(mp.rMatrices[0].val))
+        t.calcLogLike(verbose=0)
+        pf.syncChanged(t.cTree, u.cTree)
+        pf.p4_copyModelPrams(t.cTree, u.cTree)
+        pf.setPmatRoute(False)
+        decks = []
+        for w in (u, t):
+            nd = w.nodes[n.nodeNum]
+            pf.p4_setBrLen(nd.cNode, n.br.len)
+            pf.p4_calculateBigPDecks(nd.cNode)
+            decks.append([pf.p4_getBigPDeck(nd.cNode, p, mp.nGammaCat, mp.dim) for p, mp in enumerate(w.model.parts)])
+            pf.setPmatRoute(True)
+        for p, (a, b) in enumerate(zip(*decks)):
+            assert numpy.abs(a - b).max() < 1e-13, p
+            assert numpy.abs(a - old[p]).max() > 1e-6, p   # the model did change
+    finally:
+        pf.setPmatRoute(True)
+
+
 @pytest.mark.parametrize("nCat", [4, 3])
 def test_protein_category_waves_match_tile_waves(nCat):
     """The 20-state MFMA kernel with one wavefront per (tile, category)
