@@ -663,10 +663,10 @@ static void launchDeferredEach(const std::vector<DeferredP> &defer)
     (void)hipStreamSynchronize(stream());
 }
 
-// devEig: the (pi, R) snapshots and the pack were copied to the device
-// arena ahead of the P kernel on the stream (20 states: one wavefront per
-// (branch, category) would otherwise read its 3.4 KB across PCIe, 1,012
-// times for prot128, after two dependent reads of the pack)
+// devEig: the (pi, R) snapshots and the pack are copied to the device arena
+// ahead of the P kernel on the stream (20 states: one wavefront per (branch,
+// category) would otherwise read its 3.4 KB across PCIe, 1,012 times for
+// prot128, after two dependent reads of the pack)
 static bool launchParams(Tree *t, int pNum, std::vector<DeferredP> *defer = nullptr, bool devEig = false)
 {
     TreePart &tp = t->tp[pNum];
@@ -1613,11 +1613,12 @@ static bool stagePart(Tree *t, int pNum, bool full, int *nOps, std::vector<Defer
     const size_t piBytes = sizeof(double) * mp->dim;
     if (!tp.rootPiOnDevice || std::memcmp(tp.rootPiUp, tp.hRootPi, piBytes) != 0) need(tp.offPi, tp.offPi + piBytes);
     if (!tp.progOnDevice) need(tp.offProg, tp.offProg + sizeof(int) * tp.progWords);
-    // 20-state P straight from exp(Qt) for many matrices: its (pi, R)
-    // snapshots and the pack (the arena's first bytes) go up in the same
-    // copy.  A few matrices read them across PCIe sooner than a copy runs,
-    // unless a batched call's one upload launch carries them anyway.
-    const bool devEig = tp.flushDirect && mp->dim == 20 && tp.pendI > 0 && (uploads || tp.pendI * mp->nCat >= 64);
+    // P straight from exp(Qt): in a batched call its (pi, R) snapshots and the
+    // pack (the arena's first bytes) go up with the call's one upload launch;
+    // alone only for many 20-state matrices, as a few matrices, and those of
+    // 4 states, read them across PCIe sooner than a copy runs
+    const bool devEig =
+        tp.flushDirect && tp.pendI > 0 && (uploads || (mp->dim == 20 && tp.pendI * mp->nCat >= 64));
     if (devEig) need(0, tp.offPack + tp.packBytes);   // snapshots, eigen list and the pack
     if (hi > lo) {
         if (uploads)
@@ -3709,30 +3710,20 @@ double p4g_getUnconstrainedLogLike(const p4g_part *p)
 
 struct p4g_batch {
     std::vector<Tree *> trees;
-    PruneArgs *dArgs = nullptr;
-    int *dBlockItem = nullptr;
-    PruneArgs *hArgs = nullptr;
-    int *hBlockItem = nullptr;
-    int capItems = 0, capBlocks = 0;
-    // deferred 20-state direct-P flushes, read by the kernel from pinned memory
-    PmatArgs *hPm = nullptr;
-    const double **hPmIn = nullptr;
-    int *hPmFirst = nullptr;
-    int capPm = 0;
+    // one call's kernel arguments (prune args, block map, P args, P inputs,
+    // P map; callBytes), pinned and on the device
+    char *hCall = nullptr, *dCall = nullptr;
+    size_t capCall = 0;
+    int capRes = 0;
     double *hRes = nullptr;
     CopyRange *hRanges = nullptr, *dRanges = nullptr;   // program uploads (pinned)
     int capRanges = 0;
     ~p4g_batch()
     {
         hostFree(hRanges);
-        devFree(dArgs);
-        devFree(dBlockItem);
-        hostFree(hArgs);
-        hostFree(hBlockItem);
+        devFree(dCall);
+        hostFree(hCall);
         hostFree(hRes);
-        hostFree(hPm);
-        hostFree(hPmIn);
-        hostFree(hPmFirst);
     }
 };
 
@@ -3812,86 +3803,79 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
         (void)hipStreamSynchronize(stream());
         return 1;
     };
-    if (!launchUploads()) return failQueued();
-    if (!defer.empty()) {
-        // the deferred direct-P flushes in one launch per state count, before
-        // any pruning; the arrays hold the 20-state items, then the 4-state
-        const int nD = (int)defer.size();
-        if (nD > b->capPm) {
-            hostFree(b->hPm);
-            hostFree(b->hPmIn);
-            hostFree(b->hPmFirst);
-            b->capPm = 2 * nD;
-            if (!hostAlloc(&b->hPm, b->capPm, "hipHostMalloc batch P args") ||
-                !hostAlloc(&b->hPmIn, b->capPm, "hipHostMalloc batch P inputs") ||
-                !hostAlloc(&b->hPmFirst, b->capPm + 3, "hipHostMalloc batch P map")) {
-                b->capPm = 0;
-                launchDeferredEach(defer);
-                return 1;
-            }
-        }
-        PmatArgs *dPm = nullptr;
-        const double **dPmIn = nullptr;
-        int *dPmFirst = nullptr;
-        if (!hostDevPtr(b->hPm, &dPm, "device address of batch P args") ||
-            !hostDevPtr(b->hPmIn, &dPmIn, "device address of batch P inputs") ||
-            !hostDevPtr(b->hPmFirst, &dPmFirst, "device address of batch P map")) {
-            launchDeferredEach(defer);
-            return 1;
-        }
-        int q = 0, f = 0;
-        for (int dim : {20, 4}) {
-            const int q0 = q, f0 = f;
-            int total = 0;
-            for (const DeferredP &dp : defer)
-                if (dp.in && dp.a.dim == dim) {
-                    b->hPm[q] = dp.a;
-                    b->hPmIn[q] = dp.devIn ? dp.devIn : dp.in;   // the uploads ran before this launch
-                    b->hPmFirst[f++] = total;
-                    total += dp.a.nItems * dp.a.K;
-                    q++;
-                }
-            b->hPmFirst[f++] = total;
-            if (!hipOk(launchPexpMulti(dim, dPm + q0, dPmIn + q0, dPmFirst + f0, q - q0, total, stream()),
-                       "launch batched P kernel"))
-                return failQueued();
-        }
-        // the eigen route's items (after their eigensystem launches)
-        const int q0 = q, f0 = f;
-        int total = 0;
-        for (const DeferredP &dp : defer)
-            if (!dp.in) {
-                b->hPm[q] = dp.a;
-                b->hPmIn[q] = nullptr;
-                b->hPmFirst[f++] = total;
-                total += dp.a.nItems * dp.a.K * dp.a.dim * dp.a.dim;
-                q++;
-            }
-        b->hPmFirst[f++] = total;
-        if (!hipOk(launchPmatMulti(dPm + q0, dPmFirst + f0, q - q0, total, stream()), "launch batched P kernel"))
-            return failQueued();
-    }
-    const int nItems = (int)items.size();
+    // The call's kernel arguments go up in the same launch as the items'
+    // programs: every workgroup of the P and pruning kernels reads them, and
+    // from pinned memory that is a PCIe round trip in front of its work, while
+    // a copy of each array of its own is a launch each.  Measured: the 4-state
+    // P kernel 16.7 us against 46 for 64 items of 94 branches, 5.1 against
+    // 11.7 for 4 items of one branch; an MCMC generation of 4 chains and one
+    // DNA part 98 us against 108.
+    const int nItems = (int)items.size(), nD = (int)defer.size();
     int nBlocksTot = 0;
     auto itemBlocks = [](const Item &it) { return partBlocks(it.t->tp[it.p], it.t->precision); };
     for (auto &it : items) nBlocksTot += itemBlocks(it);
-    if (nItems > b->capItems) {
-        devFree(b->dArgs);
-        hostFree(b->hArgs);
-        hostFree(b->hRes);
-        b->capItems = nItems * 2;
-        if (!devAlloc(&b->dArgs, b->capItems, "hipMalloc batch args") ||
-            !hostAlloc(&b->hArgs, b->capItems, "hipHostMalloc batch args") ||
-            !hostAlloc(&b->hRes, (size_t)b->capItems * 2, "hipHostMalloc batch results"))
-            return failQueued();
+    auto up16 = [](size_t v) { return (v + 15) & ~(size_t)15; };
+    const size_t offMap = up16(sizeof(PruneArgs) * nItems), offPm = offMap + up16(sizeof(int) * 2 * nBlocksTot),
+                 offPmIn = offPm + up16(sizeof(PmatArgs) * nD), offFirst = offPmIn + up16(sizeof(double *) * nD),
+                 callBytes = offFirst + up16(sizeof(int) * (nD + 3));
+    if (callBytes > b->capCall) {
+        hostFree(b->hCall);
+        devFree(b->dCall);
+        b->capCall = 0;
+        if (!devAlloc(&b->dCall, 2 * callBytes, "hipMalloc batch args") ||
+            !hostAlloc(&b->hCall, 2 * callBytes, "hipHostMalloc batch args")) {
+            failStaged();
+            return 1;
+        }
+        b->capCall = 2 * callBytes;
     }
-    if (nBlocksTot > b->capBlocks) {
-        devFree(b->dBlockItem);
-        hostFree(b->hBlockItem);
-        b->capBlocks = nBlocksTot * 2;
-        if (!devAlloc(&b->dBlockItem, (size_t)b->capBlocks * 2, "hipMalloc batch map") ||
-            !hostAlloc(&b->hBlockItem, (size_t)b->capBlocks * 2, "hipHostMalloc batch map"))
-            return failQueued();
+    if (nItems > b->capRes) {
+        hostFree(b->hRes);
+        b->capRes = 0;
+        if (!hostAlloc(&b->hRes, (size_t)nItems * 4, "hipHostMalloc batch results")) {
+            failStaged();
+            return 1;
+        }
+        b->capRes = 2 * nItems;
+    }
+    double *dRes = nullptr;
+    char *hCallDev = nullptr;
+    if (!hostDevPtr(b->hRes, &dRes, "device address of batch results") ||
+        !hostDevPtr(b->hCall, &hCallDev, "device address of batch args")) {
+        failStaged();
+        return 1;
+    }
+    PruneArgs *const hArgs = reinterpret_cast<PruneArgs *>(b->hCall), *const dArgs = reinterpret_cast<PruneArgs *>(b->dCall);
+    int *const hMap = reinterpret_cast<int *>(b->hCall + offMap), *const dMap = reinterpret_cast<int *>(b->dCall + offMap);
+    PmatArgs *const hPm = reinterpret_cast<PmatArgs *>(b->hCall + offPm);
+    const PmatArgs *const dPm = reinterpret_cast<const PmatArgs *>(b->dCall + offPm);
+    const double **const hPmIn = reinterpret_cast<const double **>(b->hCall + offPmIn);
+    const double *const *const dPmIn = reinterpret_cast<const double *const *>(b->dCall + offPmIn);
+    int *const hFirst = reinterpret_cast<int *>(b->hCall + offFirst);
+    const int *const dFirst = reinterpret_cast<const int *>(b->dCall + offFirst);
+    // the deferred P flushes: one launch per state count of the direct route,
+    // then the eigen route's (after their eigensystem launches), each with
+    // the prefix sums of its items' matrices (eigen route: of their entries)
+    struct PLaunch {
+        int dim, q0, n, f0, total;
+    };
+    PLaunch pl[3];
+    {
+        int q = 0, f = 0;
+        for (int g = 0; g < 3; g++) {
+            PLaunch &l = pl[g];
+            l = {g == 0 ? 20 : g == 1 ? 4 : 0, q, 0, f, 0};
+            for (const DeferredP &dp : defer)
+                if (l.dim ? (dp.in && dp.a.dim == l.dim) : !dp.in) {
+                    hPm[q] = dp.a;
+                    hPmIn[q] = dp.devIn ? dp.devIn : dp.in;
+                    hFirst[f++] = l.total;
+                    l.total += dp.a.nItems * dp.a.K * (l.dim ? 1 : dp.a.dim * dp.a.dim);
+                    q++;
+                }
+            l.n = q - l.q0;
+            hFirst[f++] = l.total;
+        }
     }
     // group by (dim, precision): items of a group are contiguous in hArgs
     std::vector<int> order(nItems);
@@ -3908,17 +3892,12 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
         return ((mp->dim * 2 + prec) * 64 + kc) * 32 + wk;
     };
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return key(x) < key(y); });
-    double *dRes = nullptr;
-    if (!hostDevPtr(b->hRes, &dRes, "device address of batch results")) return failQueued();
     for (int j = 0; j < nItems; j++) {
         const Item &it = items[order[j]];
-        fillPruneArgs(it.t, it.p, it.nOps, b->hArgs[j], false);
-        b->hArgs[j].result = dRes + 2 * j;  // lnL and bad flag straight into pinned memory
+        fillPruneArgs(it.t, it.p, it.nOps, hArgs[j], false);
+        hArgs[j].result = dRes + 2 * j;  // lnL and bad flag straight into pinned memory
     }
     hipStream_t s = stream();
-    if (!hipOk(hipMemcpyAsync(b->dArgs, b->hArgs, sizeof(PruneArgs) * nItems, hipMemcpyHostToDevice, s),
-               "stage batch args"))
-        return failQueued();
     int j = 0, blk = 0;
     std::vector<std::pair<int, int>> launches;  // (first block, count) per group
     std::vector<int> groupDim, groupPrec;
@@ -3933,8 +3912,8 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
             const Item &it = items[order[jj]];
             const int nb = itemBlocks(it);
             for (int q = 0; q < nb; q++) {
-                b->hBlockItem[2 * blk] = jj;
-                b->hBlockItem[2 * blk + 1] = q;
+                hMap[2 * blk] = jj;
+                hMap[2 * blk + 1] = q;
                 blk++;
             }
             jj++;
@@ -3944,16 +3923,17 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
         groupPrec.push_back(items[order[j]].t->precision);
         groupK.push_back(items[order[j]].t->model->parts[items[order[j]].p]->nCat);
         groupAa.push_back(items[order[j]].t->tp[items[order[j]].p].mfma ? 1 : 0);
-        groupAaHbm.push_back(b->hArgs[j].aaHbm);
+        groupAaHbm.push_back(hArgs[j].aaHbm);
         {
             // the largest slot file and tip codes of the launch's 20-state items
             size_t nl = 0;
             int allTip = 1;
             for (int q = j; q < jj && groupAa.back(); q++) {
-                const PruneArgs &pa = b->hArgs[q];
+                const PruneArgs &pa = hArgs[q];
                 if (!pruneAaItemOk(pa, groupPrec.back())) {
                     setError("batch: bad 20-state program");
-                    return failQueued();
+                    failStaged();
+                    return 1;
                 }
                 nl = std::max(nl, pruneAaLdsBytes(pa.K, pa.nLds, pa.tipLds ? pa.nTax : 0, groupPrec.back()));
                 allTip &= pa.tipLds ? 1 : 0;
@@ -3972,7 +3952,7 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
             // P in LDS for the whole launch only if every item's P rows fit
             bool fits = true;
             for (int q = j; q < jj; q++) {
-                const PruneArgs &pa = b->hArgs[q];
+                const PruneArgs &pa = hArgs[q];
                 const size_t l = pruneLdsBytes(pa.nKids, pa.K, pa.dim, groupPrec.back());
                 if (!l) fits = false;
                 lds = std::max(lds, l);
@@ -3981,27 +3961,31 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
         }
         j = jj;
     }
-    if (!hipOk(hipMemcpyAsync(b->dBlockItem, b->hBlockItem, sizeof(int) * 2 * blk, hipMemcpyHostToDevice, s),
-               "stage batch map"))
-        return failQueued();
+    uploads.push_back({hCallDev, b->dCall, (unsigned long long)callBytes});
+    if (!launchUploads()) return failQueued();
+    for (const PLaunch &l : pl)
+        if (!hipOk(l.dim ? launchPexpMulti(l.dim, dPm + l.q0, dPmIn + l.q0, dFirst + l.f0, l.n, l.total, s)
+                         : launchPmatMulti(dPm + l.q0, dFirst + l.f0, l.n, l.total, s),
+                   "launch batched P kernel"))
+            return failQueued();
     // P^T of each wave item's children in program order
     for (int q = 0; q < nItems; q++) {
         const Item &it = items[order[q]];
         const TreePart &tp = it.t->tp[it.p];
         if (!tp.wave || !pruneWaveVectorP(it.t->precision)) continue;
-        const PruneArgs &pa = b->hArgs[q];
+        const PruneArgs &pa = hArgs[q];
         if (!hipOk(launchPgather(pa.PT, pa.wpre + 3 * pa.nPre, tp.nKidTot, tp.K, tp.PP, it.t->precision, s),
                    "launch P gather"))
             return failQueued();
     }
     for (size_t g = 0; g < launches.size(); g++) {
-        const int *bi = b->dBlockItem + 2 * launches[g].first;
-        const hipError_t le = groupWave[g] ? launchPruneWaveBatch(b->dArgs, bi, launches[g].second, groupK[g],
+        const int *bi = dMap + 2 * launches[g].first;
+        const hipError_t le = groupWave[g] ? launchPruneWaveBatch(dArgs, bi, launches[g].second, groupK[g],
                                                                  groupStreams[g], groupPrec[g], groupLds[g], s)
                               : groupAa[g]
-                                  ? launchPruneAaBatch(b->dArgs, bi, launches[g].second, groupK[g], groupPrec[g],
+                                  ? launchPruneAaBatch(dArgs, bi, launches[g].second, groupK[g], groupPrec[g],
                                                        groupAaHbm[g] != 0, groupAaLds[g], groupAaTip[g] != 0, s)
-                                  : launchPruneBatch(b->dArgs, bi, launches[g].second, groupDim[g], groupPrec[g],
+                                  : launchPruneBatch(dArgs, bi, launches[g].second, groupDim[g], groupPrec[g],
                                                      groupLds[g], s);
         if (!hipOk(le, "launch batched pruning kernel")) return failQueued();
     }

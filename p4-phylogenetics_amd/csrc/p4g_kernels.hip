@@ -519,7 +519,7 @@ template <int S>
 __global__ __launch_bounds__(64) void k_pexpMulti(const PmatArgs *args, const double *const *ins, const int *first,
                                                   int nItems, int total)
 {
-    // the item map (pinned host memory) is read once, in parallel, into LDS
+    // the item map is read once, in parallel, into LDS
     extern __shared__ int sFirst[];
     for (int j = threadIdx.x; j <= nItems; j += blockDim.x) sFirst[j] = first[j];
     __syncthreads();
