@@ -401,16 +401,11 @@ __device__ __forceinline__ void pruneAaBody(const PruneArgs &a, int tile, int nT
     double contrib = 0.0;
     int bad = 0;
     if (k == 0 && q == 0) {
-        auto rootE = [&](int kk) { return ((const int *)(aaSm + kk * MB))[2 * AA_TILE + pl]; };
-        int mn = SCALE ? rootE(0) : 0;
-        if (SCALE)
-            for (int kk = 1; kk < K; kk++) mn = min(mn, rootE(kk));
-        double L = 0.0;
-        for (int kk = 0; kk < K; kk++) {
-            const double Lc = ((const double *)(aaSm + kk * MB))[pl];
-            L += SCALE ? ldexp(Lc, mn - rootE(kk)) : Lc;
-        }
-        siteLogLike<SCALE>(a, L, mn, p, K, pi, contrib, bad);
+        int eL;
+        const double L = sumCategories<SCALE>(
+            K, [&](int kk) { return ((const double *)(aaSm + kk * MB))[pl]; },
+            [&](int kk) { return ((const int *)(aaSm + kk * MB))[2 * AA_TILE + pl]; }, eL);
+        siteLogLike<SCALE>(a, L, eL, p, K, pi, contrib, bad);
     }
     if (k == 0) finishSiteSumWave(a, contrib, bad, tile, nTiles);
 }

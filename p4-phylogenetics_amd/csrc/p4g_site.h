@@ -64,6 +64,24 @@ __device__ __forceinline__ void siteLogLike(const PruneArgs &a, double Lk, int e
     }
 }
 
+// A pattern's category sum, sum_k L(k) 2^-E(k), as the returned value times
+// 2^-e: e is the smallest exponent among the categories that contribute.  A
+// category whose partial became exactly 0 was not rescaled from there on, and
+// its small exponent would shift the others out of a double's range.
+template <bool SCALE, typename FL, typename FE>
+__device__ __forceinline__ double sumCategories(int K, FL L, FE E, int &e)
+{
+    constexpr int NONE = 0x7fffffff;
+    int mn = NONE;
+    if (SCALE)
+        for (int k = 0; k < K; k++)
+            if (!(L(k) == 0.0)) mn = min(mn, E(k));   // (a NaN stays in the sum)
+    e = mn == NONE ? 0 : mn;
+    double sum = 0.0;
+    for (int k = 0; k < K; k++) sum += SCALE ? ldexp(L(k), e - E(k)) : L(k);
+    return sum;
+}
+
 // A workgroup's sum and flag for the workgroup that will add them all, and
 // its ticket.  The two stores are agent-scope atomics (written through to
 // memory) and acknowledged before the ticket is drawn, which is all the

@@ -91,3 +91,81 @@ def tree_from_fixture(fx, precision="fp64"):
             n.br.parts[0].gdasrvNum = int(fx["gdasrvNums"][i]) if K > 1 else -1
     t.precision = precision
     return t
+
+
+def wide_root_cl(f):
+    """The root's partials [nCat][dim][nPat] in 80-bit floats, whose exponents
+    reach 2^-16382: site likelihoods far below a double's range stay exact.
+    P from exp(Q t), whose small entries are accurate however small t is (the
+    eigensystem leaves 1e-17 of rounding in their place)."""
+    import oracle
+    import scipy.linalg
+    K, S, nP = f.nCat, f.dim, f.patterns.shape[1]
+    Pm = numpy.zeros((len(f.parent), K, S, S), numpy.longdouble)
+    P = {}
+    for n in range(len(f.parent)):
+        if n == int(f.root):
+            continue
+        for k in range(K):
+            t = f.brLen[n] * f.rates[f.gdasrvNums[n]][k] * f.relRate / (1.0 - f.pInvar)
+            key = (int(f.rMatrixNums[n]), int(f.compNums[n]), t)
+            if key not in P:
+                P[key] = scipy.linalg.expm(oracle.bigq(f.bigR[key[0]], f.comps[key[1]]) * t)
+            Pm[n, k] = P[key]
+    kids = {}
+    for n, p in enumerate(f.parent):
+        if p >= 0:
+            kids.setdefault(int(p), []).append(n)
+    cl = {}
+    for n in f.postOrder:
+        n = int(n)
+        if n not in kids:
+            continue
+        x = numpy.ones((K, S, nP), numpy.longdouble)
+        for c in kids[n]:
+            if c in kids:
+                y = cl.pop(c)
+                x *= numpy.stack([Pm[c][k] @ y[k] for k in range(K)])
+            else:
+                code = f.patterns[f.seqNum[c]]
+                assert (code >= 0).all() and (code < S).all()
+                x *= Pm[c][:, :, code]
+        cl[n] = x
+        if n == int(f.root):
+            return x
+
+
+def wide_loglike(f):
+    """The part's lnL from wide_root_cl (no invariant sites)."""
+    assert f.pInvar == 0.0
+    pi = numpy.asarray(f.comps)[int(f.compNums[f.root])]
+    like = numpy.einsum("s,ksp->p", pi.astype(numpy.longdouble), wide_root_cl(f)) / f.nCat
+    return float((f.counts * numpy.log(like)).sum())
+
+
+def saturated_tree(dataType, nTax, nPat, nCat, alpha, precision):
+    """A balanced tree whose sites, random states mixed into conserved ones by
+    a share that grows from 0 to 1 over the patterns, are explained only by
+    the fast categories: with a very small alpha the slowest category's rate
+    is below 1e-40, so in FP32 its P is the identity and every site that
+    varies has likelihood 0 in it."""
+    from p4gpu import Data, Part, func
+    rng = numpy.random.default_rng(nTax + nPat)
+    L = ["t%d:1.0" % i for i in range(nTax)]
+    while len(L) > 3:
+        L = ["(%s,%s):0.5" % (L[i], L[i + 1]) if i + 1 < len(L) else L[i] for i in range(0, len(L), 2)]
+    t = func.readNewick("(%s);" % ",".join(L))
+    names = ["t%d" % i for i in range(nTax)]
+    t.taxNames = names
+    S = 4 if dataType == "dna" else 20
+    share = numpy.linspace(0.0, 1.0, nPat)[None, :]
+    codes = numpy.where(rng.random((nTax, nPat)) < share, rng.integers(0, S, (nTax, nPat)),
+                        rng.integers(0, S, nPat)[None, :])
+    t.data = Data(parts=[Part.fromPatterns(codes, rng.integers(1, 9, nPat), dataType)], taxNames=names)
+    t.newComp(free=1, spec="specified", val=list(rng.dirichlet(numpy.full(S, 20.0))))
+    t.newRMatrix(free=1, spec="specified", val=list(rng.lognormal(0, 0.3, S * (S - 1) // 2)))
+    t.setNGammaCat(nGammaCat=nCat)
+    t.newGdasrv(free=1, val=alpha)
+    t.setPInvar(free=0, val=0.0)
+    t.setPrecision(precision)
+    return t

@@ -9,7 +9,7 @@ import pytest
 import scipy.linalg
 
 import oracle
-from helpers import LNL_CASES, load, oracle_flat
+from helpers import LNL_CASES, load, oracle_flat, saturated_tree, wide_loglike
 
 
 # ------------------------------------------------------------------ gamma
@@ -311,3 +311,12 @@ def test_invariant_sites_known_answers():
     assert list(iv) == [1, 0, 1, 4, 1, 1]
     assert list(ia[:, 0]) == [1, 0, 0, 0] and list(ia[:, 4]) == [0, 1, 0, 0]
     assert list(ia[:, 5]) == [0, 0, 1, 0]
+
+
+@pytest.mark.parametrize("dataType", ["dna", "protein"])
+def test_wide_loglike_is_the_oracles(dataType):
+    """The 80-bit lnL that checks site likelihoods outside a double's range
+    is the oracle's where the oracle has one."""
+    f = oracle.flat_from_tree(saturated_tree(dataType, 16, 37, 4, 0.5, "fp64"), 0)
+    want = oracle.part_loglike(f)
+    assert abs(wide_loglike(f) - want) <= 1e-12 * abs(want)
