@@ -1619,11 +1619,10 @@ __device__ __forceinline__ void pruneWaveBody(const PruneArgs &a, int tile, int 
         rootE[cat][lane] = e;
         __syncthreads();
         if (wv == 0) {
-            int mn = rootE[0][lane];
-            for (int k = 1; k < K; k++) mn = min(mn, rootE[k][lane]);
-            double L = 0.0;
-            for (int k = 0; k < K; k++) L += SCALE ? ldexp(rootL[k][lane], mn - rootE[k][lane]) : rootL[k][lane];
-            siteLogLike<SCALE>(a, L, mn, p, K, pi, contrib, bad);
+            int eL;
+            const double L = sumCategories<SCALE>(
+                K, [&](int k) { return rootL[k][lane]; }, [&](int k) { return rootE[k][lane]; }, eL);
+            siteLogLike<SCALE>(a, L, eL, p, K, pi, contrib, bad);
         }
     }
     if (wv == 0) finishSiteSumWave(a, contrib, bad, tile, nTiles);
@@ -2006,11 +2005,10 @@ __device__ __forceinline__ void pruneLeanBody(const PruneArgs &a, int tile, int 
             rootE[cat][lane] = e;
             __syncthreads();
             if (cat == 0) {
-                int mn = rootE[0][lane];
-                for (int k = 1; k < K; k++) mn = min(mn, rootE[k][lane]);
-                double L = 0.0;
-                for (int k = 0; k < K; k++) L += SCALE ? ldexp(rootL[k][lane], mn - rootE[k][lane]) : rootL[k][lane];
-                siteLogLike<SCALE>(a, L, mn, p, K, pi, contrib, bad);
+                int eL;
+                const double L = sumCategories<SCALE>(
+                    K, [&](int k) { return rootL[k][lane]; }, [&](int k) { return rootE[k][lane]; }, eL);
+                siteLogLike<SCALE>(a, L, eL, p, K, pi, contrib, bad);
             }
         }
         __builtin_amdgcn_s_waitcnt(VMCNT0);

@@ -721,27 +721,34 @@ def test_protein_operands_follow_a_copy_between_precisions():
     assert rel(pf.p4_treeLogLike(b.cTree, 0), va) < FP32_TOL
 
 
-SATURATED = {"protein": [(320, 8, 0.02), (320, 4, 0.01), (244, 8, 0.02)]}
-
-
-@pytest.mark.parametrize("dataType,nTax,nCat,alpha", [(d, *c) for d, cs in SATURATED.items() for c in cs])
-def test_fp32_site_likelihoods_below_a_doubles_range(dataType, nTax, nCat, alpha):
+# (kernel: setPruneTuning's lean and wave kernels, for 4 states)
+@pytest.mark.parametrize("dataType,nTax,nCat,alpha,kernel", [
+    ("protein", 320, 8, 0.02, None), ("protein", 320, 4, 0.01, None), ("protein", 244, 8, 0.02, None),
+    ("dna", 640, 8, 0.02, -3), ("dna", 640, 4, 0.01, -3), ("dna", 640, 4, 0.01, 0), ("dna", 640, 4, 0.01, -1),
+    ("dna", 640, 4, 0.01, -2)])
+def test_fp32_site_likelihoods_below_a_doubles_range(dataType, nTax, nCat, alpha, kernel):
     """FP32 partials carry exponents, so a site likelihood of 2^-1400 has a
     logarithm; also where a category's rate is so small that the site is
     impossible in it (an exact 0, never rescaled).  Whole trees, a path after
     a branch change, and both batched, against 80-bit arithmetic."""
-    t = saturated_tree(dataType, nTax, 37, nCat, alpha, "fp32")
-    assert rel(t.calcLogLike(verbose=0), wide_loglike(oracle.flat_from_tree(t, 0))) < FP32_TOL
-    u = t.dupe()
-    u.calcLogLike(verbose=0)
-    for x, num in ((t, 5), (u, 9)):
-        n = x.nodes[num]
-        n.br.len = 0.3
-        pf.p4_setBrLen(n.cNode, n.br.len)
-        pf.p4_calculateBigPDecks(n.cNode)
-        pf.markPath(x.cTree, n.parent.nodeNum, -1)
-    got = [pf.p4_partLogLike(t.cTree, t.data.parts[0].cPart, 0, 0)]
-    pf.markAll(t.cTree, -1)
-    got += list(pf.Batch([t.cTree, u.cTree]).logLikes())
-    for x, v in zip((t, t, u), got):
-        assert rel(v, wide_loglike(oracle.flat_from_tree(x, 0))) < FP32_TOL
+    if kernel is not None:
+        pf.setPruneTuning(True, kernel, 1)
+    try:
+        t = saturated_tree(dataType, nTax, 37, nCat, alpha, "fp32")
+        assert rel(t.calcLogLike(verbose=0), wide_loglike(oracle.flat_from_tree(t, 0))) < FP32_TOL
+        u = t.dupe()
+        u.calcLogLike(verbose=0)
+        for x, num in ((t, 5), (u, 9)):
+            n = x.nodes[num]
+            n.br.len = 0.3
+            pf.p4_setBrLen(n.cNode, n.br.len)
+            pf.p4_calculateBigPDecks(n.cNode)
+            pf.markPath(x.cTree, n.parent.nodeNum, -1)
+        got = [pf.p4_partLogLike(t.cTree, t.data.parts[0].cPart, 0, 0)]
+        pf.markAll(t.cTree, -1)
+        got += list(pf.Batch([t.cTree, u.cTree]).logLikes())
+        for x, v in zip((t, t, u), got):
+            assert rel(v, wide_loglike(oracle.flat_from_tree(x, 0))) < FP32_TOL
+    finally:
+        pf.setPruneTuning(True, -3, 1)   # the library default, then the tuned choice
+        pf._applyTuning()
