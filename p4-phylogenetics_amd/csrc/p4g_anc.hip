@@ -122,18 +122,26 @@ __global__ __launch_bounds__(128) void k_ancDraw(AncArgs a)
     const size_t nPP = (size_t)a.nPatPad;
     // invariant weights present?  Without them a common power of two of the
     // variable weights cancels, so exponents are taken relative to the
-    // smallest (no underflow where the reference's unscaled values would
-    // not underflow either).
+    // smallest of the categories that contribute (no underflow where the
+    // reference's unscaled values would not underflow either; a category
+    // that is exactly 0 was not rescaled and keeps a small exponent).
     bool anyInv = false;
     if (a.pInvar != 0.0)
         for (int w = 0; w < a.nWords; w++) anyInv |= a.invMask[(size_t)w * nPP + p] != 0u;
     int Emin = 0;
     if (a.fp32 && !anyInv) {
-        Emin = 0x7fffffff;
+        constexpr int NONE = 0x7fffffff;
+        Emin = NONE;
         for (int k = 0; k < K; k++) {
             double r[SM];
-            Emin = min(Emin, rootCl<SM>(a, k, p, r));
+            const int E = rootCl<SM>(a, k, p, r);
+            bool some = false;
+#pragma unroll
+            for (int s = 0; s < SM; s++)
+                if (s < S) some |= !(r[s] == 0.0);
+            if (some) Emin = min(Emin, E);
         }
+        if (Emin == NONE) Emin = 0;
     }
     // pass 1: the table total
     double sLike = 0.0;

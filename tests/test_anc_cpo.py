@@ -17,7 +17,7 @@ import numpy
 import pytest
 
 import oracle
-from helpers import LNL_CASES, load, oracle_flat, tree_from_fixture
+from helpers import LNL_CASES, load, oracle_flat, saturated_tree, tree_from_fixture, wide_root_cl
 from p4gpu import P4Error, pf, synth
 from p4gpu.mcmc import Mcmc
 
@@ -165,6 +165,24 @@ def test_gpu_draws_match_the_oracle(case, prec):
     a, b = len(sp) // 3, len(sp) // 3 + 37
     sub = pf.drawAncStates(t.cTree, 0, a, b - a, u=u[a:b])
     assert (sub == got[a:b]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dataType,nTax,nCat,alpha", [("dna", 640, 4, 0.01), ("protein", 320, 8, 0.02)])
+def test_gpu_draws_below_a_doubles_range(dataType, nTax, nCat, alpha):
+    """FP32 draws at sites whose likelihoods go down to 2^-1415 and are exactly
+    0 in the slowest categories: the weights relative to the pattern's largest
+    from 80-bit partials.  Tolerance: two roundings of 2^-24 per taxon."""
+    t = saturated_tree(dataType, nTax, 37, nCat, alpha, "fp32")
+    t.calcLogLike(verbose=0)
+    f = oracle.flat_from_tree(t, 0)
+    cl = wide_root_cl(f)
+    cl = (cl / cl.max(axis=(0, 1))[None, None, :]).astype(float)
+    sp = numpy.repeat(numpy.arange(f.patterns.shape[1]), f.counts.astype(int))
+    u = numpy.random.default_rng(12).random(len(sp))
+    want, cum = oracle.anc_draw(f, cl, sp, u)
+    got = pf.drawAncStates(t.cTree, 0, 0, len(sp), u=u)
+    _check_draws(got, want, cum, u, 2 * nTax * 2.0 ** -24)
 
 
 @pytest.mark.gpu
