@@ -687,7 +687,7 @@ static bool launchParams(Tree *t, int pNum, std::vector<DeferredP> *defer = null
         PmatArgs a{S, K, nI, reinterpret_cast<const int *>(d + sizeof(double) * nI * K),
                    reinterpret_cast<const int *>(d + sizeof(double) * nI * K + sizeof(int) * nI),
                    reinterpret_cast<const double *>(d), tp.eigV, tp.eigVi, tp.eigLam, tp.PT64, tp.PT32,
-                   tp.PA, t->precision == FP32 ? 1 : 0};
+                   tp.PA, tp.precision == FP32 ? 1 : 0};
         const double *inDev = devEig ? reinterpret_cast<const double *>(tp.dArena) : nullptr;
         if (direct && defer) {
             defer->push_back({a, reinterpret_cast<const double *>(base), inDev});
@@ -2911,7 +2911,7 @@ int p4g_syncChanged(p4g_tree *a, p4g_tree *b)
     for (int p = 0; p < a->nParts; p++) {
         TreePart &A = a->tp[p], &B = b->tp[p];
         if (A.nSlots != B.nSlots || A.clBytes != B.clBytes || A.wave != B.wave || A.sclPerSlot != B.sclPerSlot ||
-            A.K != B.K || A.dim != B.dim) {
+            A.K != B.K || A.dim != B.dim || A.precision != B.precision) {
             setError("syncChanged: partial buffers differ");
             return 1;
         }
@@ -2928,7 +2928,7 @@ int p4g_syncChanged(p4g_tree *a, p4g_tree *b)
             if (!all && !A.chP[n] && !B.chP[n]) continue;
             r.push_back({A.PT64 + (size_t)n * pe, B.PT64 + (size_t)n * pe, pe * 8});
             if (A.PA) {
-                const bool f32 = a->precision == FP32;
+                const bool f32 = A.precision == FP32;
                 const size_t pb = (size_t)A.K * aaMatStride(f32) * (f32 ? 4 : 8);
                 r.push_back({(const char *)A.PA + n * pb, (char *)B.PA + n * pb, pb});
             } else {

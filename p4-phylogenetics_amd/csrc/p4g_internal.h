@@ -263,7 +263,7 @@ constexpr int LDS_P_BUDGET = 48 * 1024;
 struct TreePart {
     bool alloc = false;
     int dim = 0, K = 0, nPat = 0, nPatPad = 0, nSlots = 0;
-    int precision = FP64;
+    int precision = FP64;   // of the buffers (the tree's may have been set anew since they were laid out)
     // Eigen slots: [nComps*nRMat]; input pi[dim] + R[dim*dim], output
     // V[dim*dim], Vinv[dim*dim], lam[dim].
     int nEig = 0;

@@ -752,3 +752,25 @@ def test_fp32_site_likelihoods_below_a_doubles_range(dataType, nTax, nCat, alpha
     finally:
         pf.setPruneTuning(True, -3, 1)   # the library default, then the tuned choice
         pf._applyTuning()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_pending_p_matrices_outlast_a_precision_change(prec):
+    """P matrices marked before the tree's precision is set anew are computed
+    into the buffers that are there (the next evaluation lays them out again):
+    read back they are right, and after setting the precision back the
+    evaluation is the one of a tree that never left it."""
+    a, b = (synth.make_workload("prot128", seed=6, nSites=60, precision=prec)[0] for _ in range(2))
+    for t in (a, b):
+        t.calcLogLike(verbose=0)
+        for n in t.iterNodesNoRoot():
+            n.br.len *= 1.5
+            pf.p4_setBrLen(n.cNode, n.br.len)
+        pf.p4_setPrams(t.cTree, -1)
+    pf.p4_setPrecision(a.cTree, prec == "fp64")
+    nd = next(iter(a.iterNodesNoRoot()))
+    K = a.model.parts[0].nGammaCat
+    assert numpy.array_equal(pf.p4_getBigPDeck(nd.cNode, 0, K, 20),
+                             pf.p4_getBigPDeck(b.nodes[nd.nodeNum].cNode, 0, K, 20))
+    pf.p4_setPrecision(a.cTree, prec == "fp32")
+    assert pf.p4_treeLogLike(a.cTree, 0) == pf.p4_treeLogLike(b.cTree, 0)
