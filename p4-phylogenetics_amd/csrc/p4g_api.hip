@@ -3108,7 +3108,7 @@ int p4g_getCondLikes(const p4g_node *n, int pNum, double *out)
         return 1;
     }
     const int K = tp.K, S = tp.dim, nP = tp.nPat;
-    const bool f32 = t->precision == FP32;
+    const bool f32 = tp.precision == FP32;   // as they were evaluated
     std::vector<int> e;
     if (!hipOk(hipStreamSynchronize(stream()), "sync")) return 1;
     std::vector<char> raw(tp.clBytes);

@@ -774,3 +774,19 @@ def test_pending_p_matrices_outlast_a_precision_change(prec):
                              pf.p4_getBigPDeck(b.nodes[nd.nodeNum].cNode, 0, K, 20))
     pf.p4_setPrecision(a.cTree, prec == "fp32")
     assert pf.p4_treeLogLike(a.cTree, 0) == pf.p4_treeLogLike(b.cTree, 0)
+
+
+@pytest.mark.parametrize("workload", ["gtr16", "prot128"])
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_partials_read_back_after_a_precision_change(workload, prec):
+    """Setting the precision moves nothing before the next evaluation: the
+    stored partials read back as they did."""
+    t, _ = synth.make_workload(workload, seed=6, nSites=60, precision=prec)
+    t.calcLogLike(verbose=0)
+    mp = t.model.parts[0]
+    nP = len(t.data.parts[0].patterns()[1])
+    nodes = [n for n in t.iterInternals() if n is not t.root]
+    want = [pf.p4_getCondLikes(n.cNode, 0, mp.nGammaCat, mp.dim, nP) for n in nodes]
+    pf.p4_setPrecision(t.cTree, prec == "fp64")
+    for n, w in zip(nodes, want):
+        assert numpy.array_equal(pf.p4_getCondLikes(n.cNode, 0, mp.nGammaCat, mp.dim, nP), w)
