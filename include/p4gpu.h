@@ -179,9 +179,9 @@ int p4g_treeLogLike(p4g_tree *t, int getSiteLikes, double *lnL);
  * harnesses that forbid hipMalloc): p4g_treeLogLike(t, 0, lnL) computed with
  * no allocation.  The pruning kernels' reduction scratch (per-workgroup sums,
  * bad-site flags, the ticket counter) comes from one library-wide device
- * array per GPU instead of the tree's own buffers; a part needing
- * more (more than about 43,000 pattern tiles, some 700,000 patterns) is
- * rejected with an error.  The tree must already hold device state for its
+ * 8 MiB array per GPU instead of the tree's own buffers; a part needing
+ * more (beyond about 699,000 workgroups: 11 million patterns of a 20-state
+ * part, 44 million of a 4-state one) is rejected with an error.  The tree must already hold device state for its
  * current precision (one earlier p4g_treeLogLike, which allocates);
  * otherwise the call fails and allocates nothing.  Calls that overlap on
  * one GPU race on the shared array. */
@@ -368,12 +368,9 @@ void p4g_setPruneTuning(int fp32, int opsPerGroup, int stagePInLds);
  * eigensystem.  Takes effect at the next flush of pending P matrices;
  * eigensystems skipped meanwhile are recomputed when needed. */
 void p4g_setPmatRoute(int direct);
-/* Kept from the time when 20-state FP32 programs of at least minOps node ops
- * ran on a kernel of their own: one kernel now serves every 20-state program
- * of either precision, with one wavefront per (16-pattern tile, gamma
- * category), and the results do not depend on these.  They still decide from
- * which size on p4g_treeLogLikeNoAlloc refuses a 20-state FP32 part (one
- * workgroup per 16 patterns counted for such programs, per 64 otherwise). */
+/* Has no effect, and is kept for callers that still make the call: it chose
+ * between two 20-state FP32 kernels, where one kernel now serves every
+ * 20-state program of either precision. */
 void p4g_setAaTuning(int categoryWaves, int minOps);
 /* LDS cap for the 4-state program's preloaded clean children (no
  * counterpart in the reference): a dirty-path program preloads the clean

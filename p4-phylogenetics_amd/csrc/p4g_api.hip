@@ -47,10 +47,11 @@ static int g_devState = 0;  // 0 unknown, 1 ready, -1 unavailable
 // buffers.  Every GPU holds its own copy of the array until the process
 // ends; host code uses the device address that hipGetSymbolAddress returns
 // for the current device (g_scratch), never the array's name.
-constexpr size_t NOALLOC_SCRATCH_BYTES = 512 * 1024;   // the limit of one part
-// (20-state parts count fewer, larger workgroups against the limit than
-// their kernel has: at most one per 256 patterns where it has one per 16)
-static __device__ __align__(256) unsigned char scratch[16 * NOALLOC_SCRATCH_BYTES];
+// Its size is the limit of one part: 12 bytes per workgroup, some 699,000
+// workgroups (of 16 patterns in the 20-state kernel, 64 or more elsewhere:
+// 11 million patterns and more).
+constexpr size_t NOALLOC_SCRATCH_BYTES = 8 * 1024 * 1024;
+static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 constexpr int MAX_DEVICES = 64;
 static unsigned char *g_scratch[MAX_DEVICES] = {};
 
@@ -1649,18 +1650,6 @@ static int partBlocks(const TreePart &tp, int precision)
     return tp.nPatPad / (tp.wave ? pruneWaveTilePatterns(precision) : tp.mfma ? AA_TILE : pruneBlockPatterns(tp.K));
 }
 
-static int g_aaCat = 1, g_aaCatMinOps = 32;
-
-// What a 20-state part counts against the scratch limit: a workgroup per 64
-// patterns, or per 16 in FP32 programs of g_aaCatMinOps ops or more
-// (p4g_setAaTuning), and the general kernel's workgroups in FP64.  The
-// kernel itself has one per 16 patterns, which the array has room for.
-static int noAllocAaBlocks(const TreePart &tp, int precision, int nOps)
-{
-    if (precision == FP64) return tp.nPatPad / pruneBlockPatterns(tp.K);
-    return tp.nPatPad / (g_aaCat && nOps >= std::max(2, g_aaCatMinOps) ? AA_TILE : 4 * AA_TILE);
-}
-
 // Evaluate pending partials + site sum of one part (one launch).  With
 // `scr` (a device address of the no-allocation scratch array) the pruning
 // kernel's reduction scratch is taken from there, the counter is cleared by
@@ -1682,8 +1671,7 @@ static bool evalPart(Tree *t, int pNum, bool full, bool siteLikes, double *lnL, 
     if (scr) {
         // [counter, 256 B][flags int[nBlocks]][sums double[nBlocks]]
         const size_t offBad = 256, offSums = offBad + (((size_t)nBlocks * sizeof(int) + 255) & ~(size_t)255);
-        const size_t nLim = tp.mfma ? noAllocAaBlocks(tp, t->precision, nOps) : nBlocks;
-        const size_t need = 256 + ((nLim * sizeof(int) + 255) & ~(size_t)255) + nLim * sizeof(double);
+        const size_t need = offSums + (size_t)nBlocks * sizeof(double);
         if (need > NOALLOC_SCRATCH_BYTES) {
             (void)hipStreamSynchronize(s);  // queued P kernels read the staging arena
             setError("treeLogLikeNoAlloc: part " + std::to_string(pNum) + " needs " + std::to_string(need) +
@@ -2000,8 +1988,8 @@ void p4g_setPmatRoute(int direct)
 
 void p4g_setAaTuning(int categoryWaves, int minOps)
 {
-    g_aaCat = categoryWaves ? 1 : 0;
-    g_aaCatMinOps = minOps < 0 ? 0 : minOps;
+    (void)categoryWaves;
+    (void)minOps;
 }
 
 void p4g_setWavePreloadLds(int bytes) { setWavePreloadLds(bytes); }

@@ -231,15 +231,15 @@ def setWavePreloadLds(nBytes):
 
 
 def setAaLdsSlots(maxSlots):
-    """LDS slots the 20-state category kernel may forward children through
-    (default 5; 0: every child from HBM)."""
+    """LDS slots the 20-state kernel may forward children through, in either
+    precision (default 5, fewer where they would not fit; 0: every child from
+    HBM).  Same partials either way."""
     lib().p4g_setAaLdsSlots(int(maxSlots))
 
 
 def setAaTuning(categoryWaves, minOps=AA_CAT_MIN_OPS):
-    """20-state FP32 pruning with one wavefront per (tile, category) for
-    programs of at least minOps node ops (categoryWaves True, the default),
-    else one wavefront per tile."""
+    """No effect (one kernel serves every 20-state program); kept for callers
+    that still make the call."""
     lib().p4g_setAaTuning(1 if categoryWaves else 0, int(minOps))
 
 

@@ -6,7 +6,7 @@ with no device state yet is refused."""
 import numpy
 import pytest
 
-from p4gpu import P4Error, pf, synth
+from p4gpu import Data, P4Error, Part, func, pf, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +43,27 @@ def test_no_alloc_entry_point_refuses_a_tree_without_device_state():
     v = t.calcLogLike(verbose=0)
     pf.p4_setPrams(t.cTree, -1)
     assert pf.treeLogLikeNoAlloc(t.cTree) == v
+
+
+def test_no_alloc_limit_is_the_launchs_own_need():
+    """A 20-state part of 44,000 tiles: its workgroups need 0.5 MB of scratch,
+    which is there, whatever setAaTuning was told."""
+    rng = numpy.random.default_rng(24)
+    nPat, names = 44000 * 16 - 5, ["a", "b", "c", "d"]
+    t = func.readNewick("((a:0.1,b:0.2):0.05,c:0.3,d:0.1);")
+    t.taxNames = names
+    codes = rng.integers(0, 20, (4, nPat))
+    t.data = Data(parts=[Part.fromPatterns(codes, numpy.ones(nPat, int), "protein")], taxNames=names)
+    t.newComp(free=1, spec="specified", val=list(rng.dirichlet(numpy.full(20, 5.0))))
+    t.newRMatrix(free=1, spec="specified", val=list(rng.lognormal(0, 1, 190)))
+    t.setNGammaCat(nGammaCat=1)
+    t.setPInvar(free=0, val=0.0)
+    t.setPrecision("fp32")
+    want = t.calcLogLike(verbose=0)
+    try:
+        for on in (True, False):
+            pf.setAaTuning(on, 0)
+            pf.p4_setPrams(t.cTree, -1)
+            assert pf.treeLogLikeNoAlloc(t.cTree) == want
+    finally:
+        pf.setAaTuning(True)
