@@ -387,8 +387,9 @@ __global__ __launch_bounds__(64 * WAVE_MAX_K) __attribute__((amdgpu_waves_per_eu
         return Mat{*(const dvD4 *)(M + lane * 4), *(const dvD4 *)(M + 320 + (q * 4 + (pl & 3)) * 4), M[256 + lane],
                    M[384 + q * 4 + (pl & 3)]};
     };
-    const double *PA = a.PA + (size_t)cat * AA_MAT, *D = a.D + (size_t)cat * (3 * AA_MAT);
-    auto matP = [&](int node) { return PA + (size_t)node * K * AA_MAT; };
+    constexpr int PS = aaMatStride(false);   // stride of the operand table (D's matrices are packed)
+    const double *PA = a.PA + (size_t)cat * PS, *D = a.D + (size_t)cat * (3 * AA_MAT);
+    auto matP = [&](int node) { return PA + (size_t)node * K * PS; };
     auto matD = [&](int node, int which) { return D + (size_t)node * K * (3 * AA_MAT) + which * AA_MAT; };
     auto product = [&](const Mat &m, const DvPart &y) -> DvPart {
         dvD4 d0 = {0, 0, 0, 0}, d1 = {0, 0, 0, 0};

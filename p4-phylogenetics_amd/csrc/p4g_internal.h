@@ -185,11 +185,11 @@ __host__ __device__ inline int aaIndex(int s, int p, bool fp32)
     const int V = fp32 ? 4 : 2, r = s & 3, lane = (s >> 2) * 16 + p;
     return (r / V) * (64 * V) + lane * V + r % V;
 }
-// The operand table of a 20-state part, AA_MAT values per (node, category):
-// P in the order of the matrix instructions' A operands -- k-steps 0..3 of
-// the rows 0..15 by lane, k-step 4, then the same of the rows 16..19.  The
-// FP32 and FP64 instructions order their result rows differently, hence two
-// row orders.
+// The operand table of a 20-state part, AA_MAT values per (node, category),
+// aaMatStride apart: P in the order of the matrix instructions' A operands --
+// k-steps 0..3 of the rows 0..15 by lane, k-step 4, then the same of the rows
+// 16..19.  The FP32 and FP64 instructions order their result rows
+// differently, hence two row orders.
 constexpr int AA_MAT = AA_S * AA_S;
 // The table's stride: whole 128-byte lines, and the operands' parts start on
 // lines, so no two loads of a matrix touch the same line (the L1 stalls on a
@@ -272,7 +272,7 @@ struct TreePart {
     double *PT64 = nullptr;
     float *PT32 = nullptr;
     // 20-state parts of the matrix-core kernel: its operand table, float or
-    // double by precision ([nNodes][K][AA_MAT]; PT32 is not kept then)
+    // double by precision ([nNodes][K][aaMatStride]; PT32 is not kept then)
     void *PA = nullptr;
     // Partials: [nSlots][nPatPad][K][dim] of float or double, scale
     // exponents [nSlots][nPatPad] (FP32 mode); the wave kernel's layout is
