@@ -215,3 +215,42 @@ def test_derivatives_on_odd_trees(dataType, newick, nPat, nCat):
         n.br.len = t0
         assert abs(f1 - d1[n.nodeNum]) <= 1e-5 * max(1.0, abs(d1[n.nodeNum])), (n.nodeNum, f1, d1[n.nodeNum])
         assert abs(f2 - d2[n.nodeNum]) <= 1e-2 * max(1.0, abs(d2[n.nodeNum])), (n.nodeNum, f2, d2[n.nodeNum])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [52, 53, 64])
+def test_derivatives_of_many_states(S):
+    """P' and P'' of 52 states take 64 KB of LDS, of 53 and 64 (the most)
+    more than a kernel has without asking: P' = r Q P, P'' = r Q P', and the
+    likelihood across every branch is the tree's (tolerances of the tests
+    above)."""
+    import string
+    from p4gpu import Data, Part, func
+    rng = numpy.random.default_rng(S)
+    t = func.readNewick("((a:0.1,b:0.2):0.05,(c:0.3,d:0.1):0.2,e:0.15);")
+    names = ["a", "b", "c", "d", "e"]
+    t.taxNames = names
+    symbols = (string.ascii_letters + string.digits + "!$")[:S]
+    codes = numpy.where(rng.random((5, 40)) < 0.6, rng.integers(0, S, 40)[None, :], rng.integers(0, S, (5, 40)))
+    t.data = Data(parts=[Part.fromPatterns(codes, rng.integers(1, 9, 40), "standard", symbols=symbols)],
+                  taxNames=names)
+    t.newComp(free=1, spec="specified", val=list(rng.dirichlet(numpy.full(S, 20.0))))
+    t.newRMatrix(free=1, spec="specified", val=list(rng.lognormal(0, 0.3, S * (S - 1) // 2)))
+    t.setNGammaCat(nGammaCat=2)
+    t.newGdasrv(free=1, val=0.7)
+    t.setPInvar(free=0, val=0.0)
+    v = t.calcLogLike(verbose=0)
+    f = oracle.flat_from_tree(t, 0)
+    assert abs(v - oracle.part_loglike(f)) <= 1e-10 * abs(v)
+    lnl, _, _ = t.branchDerivatives()
+    Q = oracle.bigq(f.bigR[0], f.comps[0])
+    for n in t.iterNodesNoRoot():
+        assert abs(lnl[n.nodeNum] - v) <= 1e-10 * abs(v), n.nodeNum
+        P = pf.p4_getBigPDeck(n.cNode, 0, 2, S)
+        p1 = pf.p4_getBigPDeck1stD(n.cNode, 0, 2, S)
+        p2 = pf.p4_getBigPDeck2ndD(n.cNode, 0, 2, S)
+        for k in range(2):
+            r = f.rates[0][k]
+            w1, w2 = r * Q @ P[k], r * r * Q @ Q @ P[k]
+            assert numpy.abs(p1[k] - w1).max() <= 1e-12 * max(1.0, numpy.abs(w1).max()), (n.nodeNum, k)
+            assert numpy.abs(p2[k] - w2).max() <= 1e-12 * max(1.0, numpy.abs(w2).max()), (n.nodeNum, k)
