@@ -3736,7 +3736,7 @@ void p4g_freeBatch(p4g_batch *b) { delete b; }
 int p4g_batchLogLike(p4g_batch *b, double *lnL)
 {
     clearError();
-    if (!b || !lnL) return 1;
+    if (!b || !lnL || !deviceReady()) return 1;
     struct Item {
         Tree *t;
         int p, nOps, tree;
@@ -3744,30 +3744,33 @@ int p4g_batchLogLike(p4g_batch *b, double *lnL)
     std::vector<Item> items;
     std::vector<DeferredP> defer;
     std::vector<CopyRange> uploads;
+    // room for every item's upload and the call's, before anything is staged:
+    // staging clears the marks of what it lists here
+    int nRanges = 1;
+    for (const Tree *t : b->trees) nRanges += t->nParts;
+    if (nRanges > b->capRanges) {
+        hostFree(b->hRanges);
+        b->capRanges = 0;
+        const int cap = std::max(2 * nRanges, 64);
+        if (!hostAlloc(&b->hRanges, (size_t)cap, "hipHostMalloc upload ranges") ||
+            !hostDevPtr(b->hRanges, &b->dRanges, "upload ranges device address"))
+            return 1;
+        b->capRanges = cap;
+    }
     // the items' program and root-frequency uploads, in one copy launch
     auto launchUploads = [&]() -> bool {
         if (uploads.empty()) return true;
-        if ((int)uploads.size() > b->capRanges) {
-            hostFree(b->hRanges);
-            b->capRanges = 0;
-            const int cap = std::max<int>(2 * (int)uploads.size(), 64);
-            if (!hostAlloc(&b->hRanges, (size_t)cap, "hipHostMalloc upload ranges") ||
-                !hostDevPtr(b->hRanges, &b->dRanges, "upload ranges device address"))
-                return false;
-            b->capRanges = cap;
-        }
         std::copy(uploads.begin(), uploads.end(), b->hRanges);
         return hipOk(launchCopyRanges(b->dRanges, (int)uploads.size(), stream()), "launch upload kernel");
     };
     // a later item failed to stage: the items before it get their uploads and
-    // then their P matrices (whose kernels read what the uploads bring; without
-    // them only those that read the pinned arena are launched)
+    // then their P matrices (whose kernels read what the uploads bring)
     auto failStaged = [&]() {
         const std::string first = g_err;   // stays the reported error
-        if (!launchUploads())
-            defer.erase(std::remove_if(defer.begin(), defer.end(), [](const DeferredP &d) { return d.devIn != nullptr; }),
-                        defer.end());
-        launchDeferredEach(defer);
+        if (launchUploads())
+            launchDeferredEach(defer);
+        else
+            (void)hipStreamSynchronize(stream());   // queued kernels read the pinned arenas
         setError(first);
     };
     for (size_t i = 0; i < b->trees.size(); i++) {
