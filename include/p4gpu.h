@@ -365,7 +365,8 @@ void p4g_setPruneTuning(int fp32, int opsPerGroup, int stagePInLds);
  * for 4- and 20-state parts; direct = 0 uses the eigensystem (computed when
  * a slot changes) and
  * P = I + V diag(expm1(lam t)) V^-1.  Other state counts always use the
- * eigensystem.  Takes effect at the next flush of pending P matrices;
+ * eigensystem, and so, after 32 of them on an unchanged model, do the branch
+ * moves of a single 20-state tree.  Takes effect at the next flush of pending P matrices;
  * eigensystems skipped meanwhile are recomputed when needed. */
 void p4g_setPmatRoute(int direct);
 /* Has no effect, and is kept for callers that still make the call: it chose

@@ -483,6 +483,7 @@ static bool allocTreePart(Tree *t, int pNum)
         tp.dArenaHost = dah;
         tp.eigSnap.assign(tp.nEig, 0);
         tp.eigStale = false;
+        tp.branchFlushes = 0;
         tp.progOnDevice = false;
         tp.rootPiOnDevice = false;
         tp.hEigIn = reinterpret_cast<double *>(tp.hArena);
@@ -594,17 +595,31 @@ static void markP(Tree *t, int pNum, const Node *nd)
 // staging arena (no copies, no launches).  When P comes straight from the
 // (pi, R) snapshots no eigensystem is computed; the first flush on the
 // eigen route after that recomputes every slot that holds a snapshot.
-static void stageParams(Tree *t, int pNum)
+//
+// The route of 20 states: straight, but for branch moves of a single tree.
+// Straight, one matrix is a chain of products and its inputs come across
+// PCIe; from eigensystems that are there it is one short kernel (128 taxa x
+// 4,000 patterns FP32, a branch moved and its path evaluated: 42 us against 54;
+// 8 taxa x 10 patterns, one category: 31 against 43).  The eigensystems take
+// 265 us, so they are computed once AA_EIG_AFTER flushes of the same model
+// have paid for them; a flush that changes the model goes straight, and so
+// does every flush of a batched call, whose one upload brings the inputs (32
+// partitions: 14 us, and 17 from the eigensystems).
+constexpr int AA_EIG_AFTER = 32, AA_EIG_MAX_ITEMS = 15;
+static void stageParams(Tree *t, int pNum, bool batched)
 {
     TreePart &tp = t->tp[pNum];
     const int K = t->model->parts[pNum]->nCat;
     const int dim = t->model->parts[pNum]->dim;
     int nI = 0;
     for (int n = 0; n < t->nNodes; n++) nI += tp.pPending[n] ? 1 : 0;
-    // (also for the few matrices of a branch move: the direct launch over 32
-    // partitions takes 18 us where the eigen route's P kernel takes 17 and,
-    // after a change of the model, 277 for the eigensystems)
-    const bool direct = pmatDirect(dim);
+    bool direct = pmatDirect(dim);
+    if (direct && dim == AA_S) {
+        if (std::count(tp.eigPending.begin(), tp.eigPending.end(), 1) > 0)
+            tp.branchFlushes = 0;
+        else if (!batched && nI > 0 && nI <= AA_EIG_MAX_ITEMS)
+            direct = tp.eigStale && tp.branchFlushes++ < AA_EIG_AFTER;
+    }
     tp.flushDirect = direct;
     if (!direct && tp.eigStale) {
         for (int i = 0; i < tp.nEig; i++)
@@ -709,7 +724,7 @@ static bool launchParams(Tree *t, int pNum, std::vector<DeferredP> *defer = null
 // must not be written until it has run).
 static bool flushParams(Tree *t, int pNum, bool *queued = nullptr)
 {
-    stageParams(t, pNum);
+    stageParams(t, pNum, false);
     TreePart &tp = t->tp[pNum];
     if (!tp.pendE && !tp.pendI) return true;
     if (queued) *queued = true;
@@ -1604,7 +1619,7 @@ static bool stagePart(Tree *t, int pNum, bool full, int *nOps, std::vector<Defer
     // rebuilt program -- goes up in one copy of the covering range (none when
     // nothing changed); then the parameter kernels (which read the pinned
     // arena directly); the pruning launch follows on the stream
-    stageParams(t, pNum);
+    stageParams(t, pNum, uploads != nullptr);
     (void)nKids;
     size_t lo = tp.arenaBytes, hi = 0;
     auto need = [&](size_t a, size_t b) {
@@ -3006,6 +3021,7 @@ int p4g_copyModelPrams(p4g_tree *a, p4g_tree *b)
             std::memcpy(TB.hEigIn, TA.hEigIn, ne * (dim + dim * dim) * sizeof(double));
             TB.eigSnap = TA.eigSnap;
             TB.eigStale = TA.eigStale;
+            TB.branchFlushes = TA.branchFlushes;
         }
         for (int g = 0; g < A->nGdasrvs; g++)
             if (A->gdasrvs[g]->free && A->gdasrvs[g] != B->gdasrvs[g]) {

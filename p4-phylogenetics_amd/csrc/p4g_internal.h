@@ -333,6 +333,7 @@ struct TreePart {
     bool flushDirect = false;      // the staged P matrices come straight from exp(Qt)
     bool eigStale = false;         // snapshots taken while P came straight from
                                    // (pi, R), so eigV/eigVi/eigLam lag them
+    int branchFlushes = 0;         // 20 states: small flushes straight from (pi, R) since the model changed
     double *hT = nullptr;          // [nNodes][K] effective branch lengths
     int *hEs = nullptr;            // [nNodes] eigen slot of each node
     size_t packBytes = 0;

@@ -216,8 +216,9 @@ def setPruneTuning(fp32, opsPerGroup, stagePInLds):
 
 
 def setPmatRoute(direct):
-    """4-state P matrices straight from exp(Q t) (True, the default) or from
-    the eigensystem (False)."""
+    """4- and 20-state P matrices straight from exp(Q t) (True, the default;
+    repeated branch moves of a single 20-state tree still use the eigensystem)
+    or from the eigensystem (False)."""
     lib().p4g_setPmatRoute(1 if direct else 0)
 
 

@@ -790,3 +790,43 @@ def test_partials_read_back_after_a_precision_change(workload, prec):
     pf.p4_setPrecision(t.cTree, prec == "fp64")
     for n, w in zip(nodes, want):
         assert numpy.array_equal(pf.p4_getCondLikes(n.cNode, 0, mp.nGammaCat, mp.dim, nP), w)
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", FP64_TOL), ("fp32", FP32_TOL)])
+def test_p_route_of_branch_moves(prec, tol):
+    """20-state P of single branch moves straight from exp(Qt), from
+    eigensystems once there were 32 such moves, straight again after a change
+    of the model, and from the eigensystems that came with a copied model: P
+    of the moved branch and lnL against the oracle (tolerances of the tests
+    above)."""
+    t, _ = synth.make_workload("prot128", seed=9, nSites=40, precision=prec)
+    mp = t.model.parts[0]
+    K, part = mp.nGammaCat, t.data.parts[0].cPart
+    rng = numpy.random.default_rng(9)
+    nodes = list(t.iterNodesNoRoot())
+
+    def moves(x, n, check):
+        for i in range(n):
+            nd = x.nodes[nodes[int(rng.integers(len(nodes)))].nodeNum]
+            nd.br.len = float(rng.uniform(0.001, 2.0))
+            pf.p4_setBrLen(nd.cNode, nd.br.len)
+            pf.p4_calculateBigPDecks(nd.cNode)
+            pf.markPath(x.cTree, nd.parent.nodeNum, -1)
+            v = pf.p4_partLogLike(x.cTree, part, 0, 0)
+            if i % check == 0 or i == n - 1:
+                f = oracle.flat_from_tree(x, 0)
+                num = nd.nodeNum
+                want = oracle.pmat(f.bigR[f.rMatrixNums[num]], f.comps[f.compNums[num]],
+                                   nd.br.len * f.rates[f.gdasrvNums[num]] / (1.0 - f.pInvar))
+                assert numpy.abs(pf.p4_getBigPDeck(nd.cNode, 0, K, 20) - want).max() < 2e-14, i
+                assert rel(v, oracle.part_loglike(f)) < tol, i
+
+    t.calcLogLike(verbose=0)
+    moves(t, 36, 4)
+    mp.rMatrices[0].val = mp.rMatrices[0].val * numpy.linspace(0.5, 2.0, 190)
+    t.calcLogLike(verbose=0)
+    moves(t, 34, 8)
+    u = t.dupe()
+    u.calcLogLike(verbose=0)
+    pf.p4_copyModelPrams(t.cTree, u.cTree)
+    moves(u, 3, 1)
