@@ -407,7 +407,7 @@ __device__ __forceinline__ void pruneAaBody(const PruneArgs &a, int tile, int nT
     Lk += __shfl_xor(Lk, 32);
     if (q == 0) {
         ((double *)tipM)[pl] = Lk;
-        ((int *)tipM)[2 * AA_TILE + pl] = e;
+        ((int *)tipM)[2 * AA_TILE + pl] = rootExponent<SCALE>(Lk, e);
     }
     __syncthreads();
     double contrib = 0.0;

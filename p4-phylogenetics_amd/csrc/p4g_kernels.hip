@@ -1616,7 +1616,7 @@ __device__ __forceinline__ void pruneWaveBody(const PruneArgs &a, int tile, int 
             for (int s = 0; s < 4; s++) Lk += pi[s] * (double)acc[s];
         }
         rootL[cat][lane] = Lk;
-        rootE[cat][lane] = e;
+        rootE[cat][lane] = rootExponent<SCALE>(Lk, e);
         __syncthreads();
         if (wv == 0) {
             int eL;
@@ -2002,7 +2002,7 @@ __device__ __forceinline__ void pruneLeanBody(const PruneArgs &a, int tile, int 
                 for (int s = 0; s < 4; s++) Lk += pi[s] * (double)acc[s];
             }
             rootL[cat][lane] = Lk;
-            rootE[cat][lane] = e;
+            rootE[cat][lane] = rootExponent<SCALE>(Lk, e);
             __syncthreads();
             if (cat == 0) {
                 int eL;

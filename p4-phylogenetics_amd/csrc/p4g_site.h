@@ -64,19 +64,24 @@ __device__ __forceinline__ void siteLogLike(const PruneArgs &a, double Lk, int e
     }
 }
 
+// The exponent a category brings to the root's common one: e, or none if its
+// likelihood L is exactly 0.  Such a category was not rescaled from the point
+// where its partial became 0, and its small exponent would shift the others
+// out of a double's range.
+constexpr int NO_EXPONENT = 0x3fffffff;
+template <bool SCALE> __device__ __forceinline__ int rootExponent(double L, int e)
+{
+    return SCALE && L == 0.0 ? NO_EXPONENT : e;   // (a NaN keeps its place in the sum)
+}
+
 // A pattern's category sum, sum_k L(k) 2^-E(k), as the returned value times
-// 2^-e: e is the smallest exponent among the categories that contribute.  A
-// category whose partial became exactly 0 was not rescaled from there on, and
-// its small exponent would shift the others out of a double's range.
+// 2^-e; E as rootExponent gives it, e the smallest (NO_EXPONENT: the sum is 0).
 template <bool SCALE, typename FL, typename FE>
 __device__ __forceinline__ double sumCategories(int K, FL L, FE E, int &e)
 {
-    constexpr int NONE = 0x7fffffff;
-    int mn = NONE;
+    e = SCALE ? E(0) : 0;
     if (SCALE)
-        for (int k = 0; k < K; k++)
-            if (!(L(k) == 0.0)) mn = min(mn, E(k));   // (a NaN stays in the sum)
-    e = mn == NONE ? 0 : mn;
+        for (int k = 1; k < K; k++) e = min(e, E(k));
     double sum = 0.0;
     for (int k = 0; k < K; k++) sum += SCALE ? ldexp(L(k), e - E(k)) : L(k);
     return sum;
