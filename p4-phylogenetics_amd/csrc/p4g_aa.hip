@@ -184,8 +184,8 @@ __device__ __forceinline__ void pruneAaBody(const PruneArgs &a, int tile, int nT
     // The scratch matrix is written by some lanes and read by others of the
     // wave.  The hardware keeps a wave's LDS operations in order; the fence,
     // which has no instruction of its own, keeps the compiler from reordering
-    // them (an evaluation of 128 taxa x 19,877 patterns 311 us with it, 314
-    // without).
+    // them (128 taxa x 19,877 patterns FP32 313 us with it and without; four
+    // generations of 24 partitions x 4 chains 2.87 ms with and without).
     auto waveLdsFence = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
@@ -246,11 +246,14 @@ __device__ __forceinline__ void pruneAaBody(const PruneArgs &a, int tile, int nT
         v = d0;
         v4 = d1[0];
     };
+    auto loadSlot = [&](int arg, V4 &x, T &x4, int &e) {
+        loadPart(slots + arg, x, x4);
+        if (SCALE) e += *(const int *)(slots + arg + PB + (unsigned)pl * 4u);
+    };
     auto slotKid = [&](const AaKid<T> &kd, int arg, V4 &v, T &v4, int &e) {
         V4 x;
         T x4;
-        loadPart(slots + arg, x, x4);
-        if (SCALE) e += *(const int *)(slots + arg + PB + (unsigned)pl * 4u);
+        loadSlot(arg, x, x4, e);
         product(kd, x, x4, v, v4);
     };
     auto anyKid = [&](const AaKid<T> &kd, int kind, int arg, V4 &v, T &v4, int &e) {
@@ -289,13 +292,20 @@ __device__ __forceinline__ void pruneAaBody(const PruneArgs &a, int tile, int nT
         T v4;
         const int type = op.info & 3;
         if (!last && type == AA_TT) {
-            tipCol(cur[0], G ? cur[0].code : tipCode(op.arg0), acc, acc4);
-            tipCol(cur[1], G ? cur[1].code : tipCode(op.arg1), v, v4);
+            // (LDS reads that the fences of a tip's scratch need not hold up
+            // stand before it)
+            const unsigned c0 = G ? cur[0].code : tipCode(op.arg0), c1 = G ? cur[1].code : tipCode(op.arg1);
+            tipCol(cur[0], c0, acc, acc4);
+            tipCol(cur[1], c1, v, v4);
             acc *= v;
             acc4 *= v4;
         } else if (!last && type == AA_TL) {
-            tipCol(cur[0], G ? cur[0].code : tipCode(op.arg0), acc, acc4);
-            slotKid(cur[1], op.arg1, v, v4, e);
+            const unsigned c0 = G ? cur[0].code : tipCode(op.arg0);
+            V4 x;
+            T x4;
+            loadSlot(op.arg1, x, x4, e);
+            tipCol(cur[0], c0, acc, acc4);
+            product(cur[1], x, x4, v, v4);
             acc *= v;
             acc4 *= v4;
         } else if (!last && type == AA_LL) {
