@@ -93,25 +93,28 @@ def tree_from_fixture(fx, precision="fp64"):
     return t
 
 
-def wide_root_cl(f):
-    """The root's partials [nCat][dim][nPat] in 80-bit floats, whose exponents
-    reach 2^-16382: site likelihoods far below a double's range stay exact.
-    P from exp(Q t), whose small entries are accurate however small t is (the
-    eigensystem leaves 1e-17 of rounding in their place)."""
+def wide_partials(f):
+    """{node: partials [nCat][dim][nPat]} of every internal node in 80-bit
+    floats, whose exponents reach 2^-16382: site likelihoods far below a
+    double's range stay exact.  P from exp(Q t), whose small entries are
+    accurate however small t is (the eigensystem leaves 1e-17 of rounding in
+    their place)."""
     import oracle
     import scipy.linalg
     K, S, nP = f.nCat, f.dim, f.patterns.shape[1]
-    Pm = numpy.zeros((len(f.parent), K, S, S), numpy.longdouble)
     P = {}
-    for n in range(len(f.parent)):
-        if n == int(f.root):
-            continue
-        for k in range(K):
-            t = f.brLen[n] * f.rates[f.gdasrvNums[n]][k] * f.relRate / (1.0 - f.pInvar)
-            key = (int(f.rMatrixNums[n]), int(f.compNums[n]), t)
-            if key not in P:
-                P[key] = scipy.linalg.expm(oracle.bigq(f.bigR[key[0]], f.comps[key[1]]) * t)
-            Pm[n, k] = P[key]
+
+    def pmat(n, k):
+        t = f.brLen[n] * f.rates[f.gdasrvNums[n]][k] * f.relRate / (1.0 - f.pInvar)
+        key = (int(f.rMatrixNums[n]), int(f.compNums[n]), t)
+        if key not in P:
+            P[key] = scipy.linalg.expm(oracle.bigq(f.bigR[key[0]], f.comps[key[1]]) * t).astype(numpy.longdouble)
+        return P[key]
+
+    # a tip code's states: one, all (gap, '?'), or the equate's
+    tip = {c: numpy.eye(S)[c] for c in range(S)}
+    tip.update({-1: numpy.ones(S), -2: numpy.ones(S)})
+    tip.update({e - 64: numpy.asarray(row, float) for e, row in enumerate(f.equates)})
     kids = {}
     for n, p in enumerate(f.parent):
         if p >= 0:
@@ -123,16 +126,16 @@ def wide_root_cl(f):
             continue
         x = numpy.ones((K, S, nP), numpy.longdouble)
         for c in kids[n]:
-            if c in kids:
-                y = cl.pop(c)
-                x *= numpy.stack([Pm[c][k] @ y[k] for k in range(K)])
-            else:
-                code = f.patterns[f.seqNum[c]]
-                assert (code >= 0).all() and (code < S).all()
-                x *= Pm[c][:, :, code]
+            y = cl[c] if c in kids else [numpy.stack([tip[int(a)] for a in f.patterns[f.seqNum[c]]], axis=1)] * K
+            x *= numpy.stack([pmat(c, k) @ y[k] for k in range(K)])
         cl[n] = x
         if n == int(f.root):
-            return x
+            return cl
+
+
+def wide_root_cl(f):
+    """The root's partials of wide_partials."""
+    return wide_partials(f)[int(f.root)]
 
 
 def wide_loglike(f):

@@ -5,7 +5,7 @@ import numpy
 import pytest
 
 import oracle
-from helpers import LNL_CASES, load, oracle_flat, saturated_tree, tree_from_fixture, wide_loglike
+from helpers import LNL_CASES, load, oracle_flat, saturated_tree, tree_from_fixture, wide_loglike, wide_partials
 from p4gpu import Alignment, Data, P4Error, func, pf, synth
 
 pytestmark = pytest.mark.gpu
@@ -58,24 +58,16 @@ def test_golden_p_matrices(case):
 
 
 @pytest.mark.parametrize("case,prec,tol", [("het64_800", "fp64", 1e-10), ("het64_800", "fp32", 1e-4),
-                                           ("prot128_150", "fp64", 1e-10), ("prot128_150", "fp32", 1e-4),
-                                           ("prot128_150", "fp32-tile", 1e-4)])
+                                           ("prot128_150", "fp64", 1e-10), ("prot128_150", "fp32", 1e-4)])
 def test_partials_match_oracle(case, prec, tol):
     """Every stored partial, unscaled, against the oracle's: 4-state (wave
-    or lean kernel) and 20-state (FP32 on MFMA with one wavefront per
-    (tile, category), or per tile; FP64 on the grouped kernel).  The error
-    bound is relative to the largest entry of the same pattern (FP32 entries
-    far below that largest one lose relative precision, harmlessly)."""
+    or lean kernel) and 20-state (matrix cores, one wavefront per tile and
+    category).  The error bound is relative to the largest entry of the same
+    pattern (FP32 entries far below that largest one lose relative precision,
+    harmlessly)."""
     fx = load(case)
-    tile = prec == "fp32-tile"
-    prec = "fp32" if tile else prec
-    if tile:
-        pf.setAaTuning(False)
-    try:
-        t = tree_from_fixture(fx, prec)
-        t.calcLogLike(verbose=0)
-    finally:
-        pf.setAaTuning(True)
+    t = tree_from_fixture(fx, prec)
+    t.calcLogLike(verbose=0)
     f = oracle_flat(fx)
     _, _, cl = oracle.oracle_cl(f)
     K, S, nP = int(fx["nCat"]), int(fx["dim"]), f.patterns.shape[1]
@@ -88,14 +80,14 @@ def test_partials_match_oracle(case, prec, tol):
         assert (numpy.abs(got - want) <= tol * scale).all(), n.nodeNum
 
 
-@pytest.mark.parametrize("cw,slots", [(False, 5), (True, 5), (True, 2), (True, 0)])
-def test_protein_ambiguity_partials_match_oracle(cw, slots):
+@pytest.mark.parametrize("prec,slots", [("fp32", 5), ("fp32", 2), ("fp32", 0), ("fp64", 5), ("fp64", 0)])
+def test_protein_ambiguity_partials_match_oracle(prec, slots):
     """20-state tips with partial ambiguities (b = d|n, z = e|q), full ones
     (x, gaps, '?') and pInvar 0.2, on a tree whose root has three children:
-    every stored partial against the oracle's, and lnL, for the tile kernel
-    and for category waves with 5, 2 and 0 LDS slots (0: every child read
-    back from HBM).  These take the kernels' rare paths (an ambiguous tip's
-    summed P rows, HBM children, a third root child)."""
+    every stored partial against 80-bit ones, and lnL, with 5, 2 and 0 LDS
+    slots (0: every child read back from HBM).  These take the kernel's rare
+    paths (an ambiguous tip's summed columns, HBM children, a third root
+    child)."""
     fx = dict(load("prot128_150"))
     rng = numpy.random.default_rng(11)
     pat = fx["patterns"].copy()
@@ -106,23 +98,23 @@ def test_protein_ambiguity_partials_match_oracle(cw, slots):
     fx["pInvar"] = numpy.array(0.2)
     assert int((fx["parent"] == int(fx["root"])).sum()) == 3
     f = oracle_flat(fx)
-    wantL, _, cl = oracle.oracle_cl(f)
+    # (with P from exp(Qt): the oracle's own, from the eigensystem, leaves up
+    # to 7e-10 in partials that hang on P's smallest entries)
+    wantL, cl = oracle.part_loglike(f), wide_partials(f)
     K, S, nP = int(fx["nCat"]), int(fx["dim"]), f.patterns.shape[1]
     try:
-        pf.setAaTuning(cw, 0)
         pf.setAaLdsSlots(slots)
-        t = tree_from_fixture(fx, "fp32")
+        t = tree_from_fixture(fx, prec)
         v = t.calcLogLike(verbose=0)
         got = {n.nodeNum: pf.p4_getCondLikes(n.cNode, 0, K, S, nP) for n in t.nodes
                if not (n.isLeaf or n is t.root)}
     finally:
-        pf.setAaTuning(True)
         pf.setAaLdsSlots(5)
-    assert rel(v, wantL) < FP32_TOL, (v, wantL)
+    assert rel(v, wantL) < (FP32_TOL if prec == "fp32" else FP64_TOL), (v, wantL)
     for num, g in got.items():
         want = cl[num]
         scale = want.max(axis=(0, 1))[None, None, :]
-        assert (numpy.abs(g - want) <= 1e-4 * scale).all(), num
+        assert (numpy.abs(g - want) <= (1e-4 if prec == "fp32" else 1e-10) * scale).all(), num
 
 
 # -------------------------------------------------- full-size workloads
@@ -473,44 +465,49 @@ def test_copied_model_serves_the_eigen_route(stale):
         pf.setPmatRoute(True)
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("nCat", [4, 3])
-def test_protein_category_waves_match_tile_waves(nCat):
-    """The 20-state MFMA kernel with one wavefront per (tile, category)
-    stores the same partials and exponents, bit for bit, as the one with a
-    wavefront per tile holding every category; lnL agrees to 1e-12 (only
-    the FP64 root sum over categories is added in another order) and with
-    the FP64 path to the FP32 tolerance.  nCat 3: 192-thread workgroups."""
+def test_protein_program_shapes_give_the_same_partials(nCat, prec):
+    """However a 20-state program hands a child on -- through an LDS slot,
+    written to HBM and read back, or left in HBM by an earlier evaluation (a
+    dirty path) -- the partials are the same, bit for bit, and lnL to 1e-12.
+    nCat 3: 192-thread workgroups."""
     fx = dict(load("prot128_150"))
     fx["nCat"] = numpy.array(nCat)
     K, S, nP = nCat, int(fx["dim"]), fx["patterns"].shape[1]
     want = tree_from_fixture(fx, "fp64").calcLogLike(verbose=0)
     if nCat == 4:
         assert rel(want, float(fx["lnL"])) < FP64_TOL
+
+    def partials(t):
+        return [pf.p4_getCondLikes(n.cNode, 0, K, S, nP) for n in t.nodes if not (n.isLeaf or n is t.root)]
+
     res = {}
     try:
-        # tile waves; category waves with children from HBM; category waves
-        # forwarding children through the LDS slot file (the default)
-        for cw, slots in ((False, 5), (True, 0), (True, 5), (True, 2)):
-            pf.setAaTuning(cw, 0)
+        for slots in (0, 5, 2):
             pf.setAaLdsSlots(slots)
-            t = tree_from_fixture(fx, "fp32")
+            t = tree_from_fixture(fx, prec)
             v = t.calcLogLike(verbose=0)
-            assert rel(v, want) < FP32_TOL, (cw, slots, v, want)
-            cls = [pf.p4_getCondLikes(n.cNode, 0, K, S, nP) for n in t.nodes if not (n.isLeaf or n is t.root)]
-            res[(cw, slots)] = (v, cls)
+            assert rel(v, want) < (FP32_TOL if prec == "fp32" else FP64_TOL), (slots, v, want)
+            res[slots] = (v, partials(t))
+            # every path from a leaf again, most of its children clean
+            for n in t.iterLeavesNoRoot():
+                pf.markPath(t.cTree, n.parent.nodeNum, -1)
+                w = pf.p4_partLogLike(t.cTree, t.data.parts[0].cPart, 0, 0)
+                assert rel(w, v) < 1e-12, (slots, n.nodeNum)
+            res[slots, "paths"] = (w, partials(t))
     finally:
-        pf.setAaTuning(True)
         pf.setAaLdsSlots(5)
-    for key in ((True, 0), (True, 5), (True, 2)):
-        assert rel(res[key][0], res[(False, 5)][0]) < 1e-12, key
-        for a, b in zip(res[key][1], res[(False, 5)][1]):
+    for key in res:
+        assert rel(res[key][0], res[0][0]) < 1e-12, key
+        for a, b in zip(res[key][1], res[0][1]):
             assert numpy.array_equal(a, b), key
 
 
 def test_batch_mixes_protein_kernels():
-    """One batched call where one tree's protein parts run long programs
-    (category waves) and another's short dirty paths (tile kernel): every
-    lnL equals the tree's full evaluation."""
+    """One batched call where one tree's protein parts run full programs and
+    another's dirty paths, which read clean children from HBM (the kernel's
+    two instances): every lnL equals the tree's full evaluation."""
     trees = [synth.make_workload("multi48", seed=s, nSites=1500, precision="fp32")[0] for s in (6, 7)]
     want = [t.calcLogLike(verbose=0) for t in trees]
     for n in trees[0].iterInternals():
@@ -573,11 +570,12 @@ def test_batch_direct_p_in_one_launch():
         assert dims == {4, 20}
 
 
-def test_batch_eigen_route_p_in_one_launch():
-    """A branch move on every chain of a multi-partition batch: 20-state
-    parts recompute that branch's P on the eigen route (a flush of few
-    matrices), all items in one launch; P decks equal, bit for bit, and lnL
-    agrees with the same trees evaluated one by one."""
+@pytest.mark.parametrize("direct", [True, False])
+def test_batch_branch_move_p_in_one_launch(direct):
+    """A branch move on every chain of a multi-partition batch: that branch's
+    P straight from exp(Qt) (one launch per state count) or from the
+    eigensystems (one launch for all items); P decks equal, bit for bit, and
+    lnL agrees with the same trees evaluated one by one."""
     def make():
         return [synth.make_workload("multi48", seed=s, nSites=1500, precision="fp32")[0] for s in (11, 12)]
 
@@ -592,24 +590,28 @@ def test_batch_eigen_route_p_in_one_launch():
             m = m.parent
         return n.nodeNum
 
-    A, B = make(), make()
-    for t in A + B:
-        t.calcLogLike(verbose=0)
-    moved = [move(t) for t in A]
-    for t in B:
-        move(t)
-    got = pf.Batch([t.cTree for t in A]).logLikes()
-    want = [pf.p4_treeLogLike(t.cTree, 0) for t in B]
-    for g, w in zip(got, want):
-        assert rel(g, w) < 1e-12, (g, w)
-    for ta, tb, nn in zip(A, B, moved):
-        dims = set()
-        for p, mp in enumerate(ta.model.parts):
-            pa = pf.p4_getBigPDeck(ta.nodes[nn].cNode, p, mp.nGammaCat, mp.dim)
-            pb = pf.p4_getBigPDeck(tb.nodes[nn].cNode, p, mp.nGammaCat, mp.dim)
-            assert numpy.array_equal(pa, pb), (p, nn)
-            dims.add(mp.dim)
-        assert dims == {4, 20}
+    pf.setPmatRoute(direct)
+    try:
+        A, B = make(), make()
+        for t in A + B:
+            t.calcLogLike(verbose=0)
+        moved = [move(t) for t in A]
+        for t in B:
+            move(t)
+        got = pf.Batch([t.cTree for t in A]).logLikes()
+        want = [pf.p4_treeLogLike(t.cTree, 0) for t in B]
+        for g, w in zip(got, want):
+            assert rel(g, w) < 1e-12, (g, w)
+        for ta, tb, nn in zip(A, B, moved):
+            dims = set()
+            for p, mp in enumerate(ta.model.parts):
+                pa = pf.p4_getBigPDeck(ta.nodes[nn].cNode, p, mp.nGammaCat, mp.dim)
+                pb = pf.p4_getBigPDeck(tb.nodes[nn].cNode, p, mp.nGammaCat, mp.dim)
+                assert numpy.array_equal(pa, pb), (p, nn)
+                dims.add(mp.dim)
+            assert dims == {4, 20}
+    finally:
+        pf.setPmatRoute(True)
 
 
 def test_batch_error_keeps_staged_p_matrices():
