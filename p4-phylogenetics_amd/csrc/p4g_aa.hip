@@ -72,9 +72,9 @@ template <typename T> struct AaKid {
 // (Sethi-Ullman order, see buildAaProgram) and always to HBM, where later
 // evaluations read them.  There is no barrier in the chain: FP32 scale
 // exponents are per (node, pattern, category), combined exactly at the root.
-// Measured: 128 taxa, 19,877 patterns, 4 categories, FP32 300 us (430 with a
+// Measured: 128 taxa, 19,877 patterns, 4 categories, FP32 300-322 us (430 with a
 // barrier per op for a shared exponent, tip rows gathered from memory and
-// loads waiting for stores); 48 taxa x 5,003 patterns FP64 80 us (1,124 on
+// loads waiting for stores); 48 taxa x 5,003 patterns FP64 77 us (1,124 on
 // the general kernel, one lane per pattern and category).  The floors are
 // the partials' stores (156 and 28 us at the rate of a large copy) and the
 // padded matrix products (85 and 24 us).  What is left is issue: with the

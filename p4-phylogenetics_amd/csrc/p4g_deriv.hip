@@ -345,7 +345,7 @@ __global__ __launch_bounds__(64 * WAVE_MAX_K) void k_edgeDerivs4(DerivArgs a)
 // of pattern p, register 4 state 16 + q.  Bound by the products: per node
 // with two children up to seven (its P^T, and P, P' and P'' of each internal
 // child), each ten v_mfma_f64_16x16x4f64 with the 20 rows padded to 32.
-// 48 taxa x 2,003 patterns, 4 categories: 216 us (one lane per pattern and
+// 48 taxa x 2,003 patterns, 4 categories: 217 us (one lane per pattern and
 // category, with register arrays in scratch memory: 10.2 ms).
 struct DvPart {
     dvD4 x;
